@@ -61,6 +61,15 @@ constexpr int kWaves = 4;
 #ifndef ANEDVD_SMALL_MEAN
 #define ANEDVD_SMALL_MEAN 64
 #endif
+// Mean group size from which the decode kernels take 32-token chunks (two 16-token
+// tiles, the second skipped where a group has no tokens for it): most groups then
+// hold more than 16 tokens or nearly so, and each pass over an expert's weights serves
+// them all.  One box, 16- against 32-token chunks (us): Qwen3 Q8_0 mean 8 136.7 / 137.9,
+// mean 10 145.6 / 142.0, mean 16 200 / 161, mean 21 248 / 177; Q4_K_M mean 8 109.7 /
+// 113.8, mean 12 131.7 / 129.9, mean 21 205 / 156; Mixtral Q4_0 mean 10 203.2 / 204.4,
+// mean 25 368 / 281.  (64-token chunks: Qwen3 Q8_0 mean 21 186, the accumulators and
+// activations then leave one or two wavefronts per SIMD.)
+constexpr int kWideMean = 10;
 constexpr int kCUs = 256;  // MI355X compute units
 #ifdef ANEDVD_MM_WPE
 #define MM_ATTR __attribute__((amdgpu_waves_per_eu(ANEDVD_MM_WPE)))
@@ -499,8 +508,8 @@ struct AOpL {
     int s0;
 };
 
-template <int MT, int MODE>
-__device__ inline void load_a(AStep<MT, MODE> &x, const AOpL<MT> &a, int s)
+template <int MT, int MODE, int TA>
+__device__ inline void load_a(AStep<MT, MODE> &x, const AOpL<TA> &a, int s)
 {
     const int o = (s - a.s0) * 2 * kStep;
 #pragma unroll
@@ -510,12 +519,12 @@ __device__ inline void load_a(AStep<MT, MODE> &x, const AOpL<MT> &a, int s)
     }
     if (MODE == kStepDs) {
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) x.dv[mt] = *(const f32x4 *)(a.ds + (s - a.s0) * 16 * MT + a.doff[mt]);
+        for (int mt = 0; mt < MT; mt++) x.dv[mt] = *(const f32x4 *)(a.ds + (s - a.s0) * 16 * TA + a.doff[mt]);
     }
 }
 
-template <int MT, int MODE>
-__device__ inline void load_a(AStep<MT, MODE> &x, const AOp<MT> &a, int s)
+template <int MT, int MODE, int TA>
+__device__ inline void load_a(AStep<MT, MODE> &x, const AOp<TA> &a, int s)
 {
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
@@ -638,6 +647,20 @@ __device__ inline void mm_steps(const Planes &W, int rb, int s0, int s1, int lan
     }
 }
 
+// mm_steps over the chunk's live 16-token tiles only: a chunk of at most 16 tokens
+// in a 32-token kernel runs one tile (uniform over the workgroup).
+template <class D, int MT, int MODE, class AS>
+__device__ inline void mm_live(const Planes &W, int rb, int s0, int s1, int lane, const AS &A, f32x4 (*acc)[4], int nt)
+{
+    if constexpr (MT > 1) {
+        if (nt <= 16 * (MT - 1)) {
+            mm_live<D, MT - 1, MODE>(W, rb, s0, s1, lane, A, acc, nt);
+            return;
+        }
+    }
+    mm_steps<D, MT, MODE>(W, rb, s0, s1, lane, A, acc);
+}
+
 struct MmArgs {
     QMat w0, w1;     // gate and up (gate/up), or down (w0)
     ActQ x;          // input activations: tokens (gate/up) or positions (down)
@@ -702,7 +725,7 @@ __global__ __launch_bounds__(256) MM_ATTR void k_mm_gateup(MmArgs a)
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int t = 0; t < 4; t++) acc[mt][t] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-    mm_steps<D, MT, kRow>(W, rb, ub * D::kSpu, ue * D::kSpu, lane, A, acc);
+    mm_live<D, MT, kRow>(W, rb, ub * D::kSpu, ue * D::kSpu, lane, A, acc, nt);
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
@@ -876,7 +899,7 @@ __global__ __launch_bounds__(256) MM_ATTR void k_mm_down(MmArgs a)
             A.qoff[mt] = (16 * mt + n) * rowb + 32 * gq;
             A.doff[mt] = 16 * mt + 4 * gq;
         }
-        mm_steps<D, MT, kStepDs>(W, rb, s0, s0 + sw, lane, A, acc);
+        mm_live<D, MT, kStepDs>(W, rb, s0, s0 + sw, lane, A, acc, nt);
     } else {
         if (rb >= a.H / kRowBlock) return;  // no barriers in this kernel
         AOp<MT> A;
@@ -888,7 +911,7 @@ __global__ __launch_bounds__(256) MM_ATTR void k_mm_down(MmArgs a)
             A.qoff[mt] = (p0 + 16 * mt + n) * a.I * 2 + 32 * gq;
             A.doff[mt] = (p0 + 16 * mt + 4 * gq) * 4;
         }
-        mm_steps<D, MT, kStepDs>(W, rb, u0 * D::kSpu, (u0 + upw) * D::kSpu, lane, A, acc);
+        mm_live<D, MT, kStepDs>(W, rb, u0 * D::kSpu, (u0 + upw) * D::kSpu, lane, A, acc, nt);
     }
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
@@ -1048,11 +1071,11 @@ static int steps_per_unit(int type) { return tile_fmt(type).spu; }
 // Dynamic LDS of a kPart down workgroup: 16 rows of its steps in the activation
 // format, and a descale per (step, row).
 constexpr size_t kFuseLdsMax = 64 * 1024;
-static size_t down_part_lds(int down_type, int I, int ks_dn)
+static size_t down_part_lds(int down_type, int I, int ks_dn, int mt)
 {
     const int spu = steps_per_unit(down_type);
     const size_t sw = (size_t)(I / kStep / spu / ks_dn) * spu;
-    return 16 * sw * 2 * kStep + sw * 16 * 4;
+    return mt * (16 * sw * 2 * kStep + sw * 16 * 4);
 }
 
 bool mm_supported(int type) { return tile_fmt(type).qb != 0; }
@@ -1080,8 +1103,8 @@ MmPlan plan_mm(int gate_type, int down_type, int H, int I, int P, int max_u, int
     // The grouped GEMM (64-token chunks of a group, activations staged in LDS and
     // shared by four wavefronts) once the groups average 32 tokens and its gate/up
     // grid has a workgroup per CU at least; the chunks then give the grid its
-    // parallelism and K is not split.  Below that, the decode kernels: 16-token
-    // tiles, activations straight from L2, K split over workgroups.  (A single
+    // parallelism and K is not split.  Below that, the decode kernels: chunks of one
+    // or two 16-token tiles, activations straight from L2, K split over workgroups.  (A single
     // shared expert at 32 tokens on the grouped GEMM would be 22 workgroups: it
     // measured 105 us against the decode kernels' split K.  Kernels that read the
     // activations from L2 per wavefront with folded scales and 32- or 64-token
@@ -1114,7 +1137,7 @@ MmPlan plan_mm(int gate_type, int down_type, int H, int I, int P, int max_u, int
         p.nsmall = p.small ? max_u : 0;
     } else {
         p.kind = kMmDecode;
-        p.mt = 1;
+        p.mt = mean >= kWideMean ? 2 : 1;
     }
     p.chunk = 16 * p.mt;
     p.nchunk = P / p.chunk + max_u;
@@ -1136,7 +1159,7 @@ MmPlan plan_mm(int gate_type, int down_type, int H, int I, int P, int max_u, int
     // even if every token of the call sends a slot to the same expert (a chunk
     // holds at most min(T, 16) tokens).  Otherwise k_act_reduce finishes them.
     const int sw = I / kStep / steps_per_unit(down_type) / p.ks_dn * steps_per_unit(down_type);
-    p.fuse = p.ks_gu > 1 && down_part_lds(down_type, I, p.ks_dn) <= kFuseLdsMax && std::min(T, 16) * sw <= 64;
+    p.fuse = p.ks_gu > 1 && down_part_lds(down_type, I, p.ks_dn, p.mt) <= kFuseLdsMax && std::min(T, p.chunk) * sw <= 64;
     return p;
 }
 
@@ -1154,10 +1177,9 @@ static int launch_gateup_t(const MmArgs &a, hipStream_t st)
 template <class D, int MT>
 static int launch_down_t(const MmArgs &a, hipStream_t st)
 {
-    static_assert(MT == 1, "the kPart LDS budget is sized for 16-token chunks");
     const size_t wgs = (size_t)a.nchunk * ((a.H / kRowBlock + kWaves - 1) / kWaves) * a.KS;
     if (a.KSg > 1) {
-        const size_t lds = down_part_lds(a.w0.type, a.I, a.KS);
+        const size_t lds = down_part_lds(a.w0.type, a.I, a.KS, MT);
         hipLaunchKernelGGL((k_mm_down<D, MT, true>), dim3((unsigned)wgs), dim3(256), lds, st, a);
     } else {
         hipLaunchKernelGGL((k_mm_down<D, MT, false>), dim3((unsigned)wgs), dim3(256), 0, st, a);
@@ -1167,15 +1189,15 @@ static int launch_down_t(const MmArgs &a, hipStream_t st)
 }
 
 template <class D>
-static int launch_gateup_d(const MmArgs &a, int, hipStream_t st)
+static int launch_gateup_d(const MmArgs &a, int mt, hipStream_t st)
 {
-    return launch_gateup_t<D, 1>(a, st);
+    return mt == 2 ? launch_gateup_t<D, 2>(a, st) : launch_gateup_t<D, 1>(a, st);
 }
 
 template <class D>
-static int launch_down_d(const MmArgs &a, int, hipStream_t st)
+static int launch_down_d(const MmArgs &a, int mt, hipStream_t st)
 {
-    return launch_down_t<D, 1>(a, st);
+    return mt == 2 ? launch_down_t<D, 2>(a, st) : launch_down_t<D, 1>(a, st);
 }
 
 int launch_expert_gateup(const QMat &gate, const QMat &up, const ActQ &x, int H, int I, const Dispatch &d, int P,

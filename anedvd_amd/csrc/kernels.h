@@ -90,14 +90,14 @@ int launch_act_prep(const float *d_x, int rows, int K, const ActQ &xq, hipStream
 
 // k_mm.hip -- expert products on MFMA
 enum MmKind {
-    kMmDecode = 0,   // k_mm_gateup / k_mm_down: 16-token tiles, per-block f32 scales, K split
+    kMmDecode = 0,   // k_mm_gateup / k_mm_down: one or two 16-token tiles, per-block f32 scales, K split
     kMmStaged = 1    // k_pf_gateup / k_pf_down: 64-token chunks, activations staged in LDS
 };
 struct MmPlan {
     int kind;     // MmKind
     int ks_gu;    // K split of gate/up (workgroups per 64-row block)
     int ks_dn;    // K split of down
-    int mt;       // 16-token tiles per chunk: 1 (decode), 4 or 8 (grouped GEMM)
+    int mt;       // 16-token tiles per chunk: 1 or 2 (decode), 4 or 8 (grouped GEMM)
     int mt_gu;    // grouped GEMM: 16-token tiles per gate/up workgroup (4 or 8, at most mt)
     int mt_dn;    // grouped GEMM: 16-token tiles per down workgroup (4 or 8, at most mt)
     int contig;   // grouped GEMM: XCD-contiguous workgroup order

@@ -427,6 +427,21 @@ def test_forward_grouped_every_live_tile_count(ctx, types):
     assert st["chunk"] == (128 if wide_gu or wide_dn else 64)  # gate/up and down pick their widths apart
 
 
+@pytest.mark.parametrize("shape", [(1024, 512), (256, 8192)], ids=["k-split", "whole-k"])
+@pytest.mark.parametrize("types", FORMATS, ids=lambda t: "/".join(W.TYPE_NAMES[x] for x in t))
+def test_forward_decode_32_token_chunks(ctx, types, shape):
+    """The decode kernels' 32-token chunks (mean group 18): groups at the edges of one
+    and two 16-token tiles and of a second chunk, with gate/up's K split (finished in
+    the down kernel) and whole."""
+    sizes = [1, 15, 16, 17, 31, 32, 33, 3]
+    lg = _logits_for_groups(sizes, seed=31)
+    spec = dataclasses.replace(W.MIXTRAL_8X7B_Q4_0, name="mm-32", hidden=shape[0], inter=shape[1],
+                               gate_type=types[0], up_type=types[1], down_type=types[2], scale_sigma=0.01)
+    _, _, err, st = _forward_case(ctx, spec, lg.shape[0], seed=31, logits=lg)
+    assert err <= REL_L2_TOL
+    assert st["path"] == 0 and st["chunk"] == 32 and st["max_group"] == max(sizes)
+
+
 @pytest.mark.parametrize("types", [(W.Q4_0, W.Q4_0, W.Q4_0), (W.Q4_K, W.Q4_K, W.Q6_K), (W.Q8_0, W.Q8_0, W.Q5_K)],
                          ids=lambda t: "/".join(W.TYPE_NAMES[x] for x in t))
 def test_forward_grouped_split_k_down(ctx, types):
