@@ -70,6 +70,10 @@ constexpr int kWaves = 4;
 // mean 25 368 / 281.  (64-token chunks: Qwen3 Q8_0 mean 21 186, the accumulators and
 // activations then leave one or two wavefronts per SIMD.)
 constexpr int kWideMean = 10;
+// Mean group size from which the decode kernels stage their activations (ASource):
+// with fewer tokens per group a direct load touches few lines anyway.
+constexpr int kStageMean = 2;
+static_assert(kStageMean <= kWideMean, "32-token chunks are staged");
 constexpr int kCUs = 256;  // MI355X compute units
 #ifdef ANEDVD_MM_WPE
 #define MM_ATTR __attribute__((amdgpu_waves_per_eu(ANEDVD_MM_WPE)))
@@ -478,23 +482,84 @@ struct MQ6_K {
 //         consecutive positions -- come in with one 16-byte load per token tile.
 enum DsMode { kRow, kStepDs };
 
+// A wavefront's activations of one step.  A lane's MFMA operand is a 16-byte piece of
+// token row l % 16, so neighbouring lanes read different rows: loaded that way (kASelf)
+// a 16-byte load touches as many cache lines as the tile has tokens, and these lookups,
+// not the bytes, bounded the 32-token chunks (all lanes on one row: Qwen3 Q8_0 333
+// tokens 177 -> 156 us, Mixtral Q4_0 100 tokens 281 -> 206 us, in a timing copy).
+// Staged (kAStaged), a load takes 8 whole rows of the step's 64 columns, 8 lanes a
+// row, and the wavefront turns them into operands through LDS of its own (kStageBytes
+// per token tile, no barrier: one wavefront's LDS accesses are done in order).  Row r's
+// 16-byte piece p sits at piece p ^ a_sw(r), so reads and writes of 8 consecutive lanes
+// hit distinct banks.  Measured (us, one box, self / staged): Qwen3 Q8_0 333 tokens
+// 176.8 / 171.3, DeepSeek-V2-Lite 256 206 / 196.5, Mixtral 100 279 / 246.5, Qwen3 Q4_K_M
+// 128 108.7 / 106.1, Q8_0 32 114.2 / 113.1; groups of one token are better off without
+// (Mixtral one token 55.4 / 56.0).
+enum ASource { kASelf, kAStaged, kAPart };  // kAPart: AOpL below
+constexpr int kStageBytes = 16 * 2 * kStep;  // LDS of one 16-token tile's step
+
+__device__ inline int a_sw(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+
 template <int MT, int MODE>
 struct AStep {
-    half8 a0[MT], a1[MT];
+    u32x4 raw[2 * MT];  // load i: the lane's piece of row 8 i + l / 8
     f32x4 dv[MODE == kStepDs ? MT : 1];
 };
 
-// Where a lane's activations come from: its A row's byte offset (token l % 16 of
-// tile mt, plus lane group g's 32 bytes) in the f16 values and, for kStepDs, the
-// byte offset of its first result token's descale within a group (ld4 bytes per
-// group).
-template <int MT>
+// Where they come from: the byte offsets of the lane's pieces and, for kStepDs, of its
+// first result token's descale in tile mt (ld4 bytes per group); where they go.
+template <int MT, bool kStage>
 struct AOp {
     rsrc_t q, ds;
-    int qoff[MT];
+    int qoff[2 * MT];  // staged: load i's; else tile mt's at 2 mt
     int doff[MT];
     int ld4;
+    char *st;  // the wavefront's LDS
+    int wr;    // the lane's byte for load 0 (load i: + 1024 i, odd ones ^ 16)
+    int rd;    // the lane's operand of block 0 in tile 0 (block 1: ^ 16; tile mt: + kStageBytes mt)
+    __device__ inline void stage_at(char *lds, int lane)
+    {
+        const int r = lane >> 3, n = lane & 15;
+        st = lds;
+        wr = r * 128 + (((lane & 7) ^ a_sw(r)) << 4);
+        rd = n * 128 + (((2 * (lane >> 4)) ^ a_sw(n)) << 4);
+    }
 };
+
+template <int MT, int MODE, int TA, bool kStage>
+__device__ inline void load_a(AStep<MT, MODE> &x, const AOp<TA, kStage> &a, int s)
+{
+#pragma unroll
+    for (int i = 0; i < 2 * MT; i++)
+        x.raw[i] = __builtin_amdgcn_raw_buffer_load_b128(a.q, a.qoff[kStage ? i : i & ~1],
+                                                         s * 2 * kStep + (kStage ? 0 : 16 * (i & 1)), 0);
+    if (MODE == kStepDs) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(a.ds, a.doff[mt], s * a.ld4, 0);
+            __builtin_memcpy(&x.dv[mt], &v, 16);
+        }
+    }
+}
+
+// Puts a loaded step where the operands are read from (the step before it is done).
+template <int MT, int MODE, int TA, bool kStage>
+__device__ inline void publish_a(const AStep<MT, MODE> &x, const AOp<TA, kStage> &a)
+{
+    if constexpr (!kStage) return;
+#pragma unroll
+    for (int i = 0; i < 2 * MT; i++) *(u32x4 *)(a.st + 1024 * i + ((i & 1) ? a.wr ^ 16 : a.wr)) = x.raw[i];
+}
+
+template <int MT, int MODE, int TA, bool kStage>
+__device__ inline void operand_a(half8 *av, const AStep<MT, MODE> &x, const AOp<TA, kStage> &a, int j)
+{
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+        if constexpr (kStage) av[mt] = *(const half8 *)(a.st + kStageBytes * mt + (j ? a.rd ^ 16 : a.rd));
+        else av[mt] = as_h8(x.raw[2 * mt + j]);
+    }
+}
 
 // The same operands from LDS: the fused-reduce down kernel's prologue writes its
 // 16 MT rows there, for its steps [s0, s0 + n) only (rows of rowb bytes in the
@@ -514,8 +579,8 @@ __device__ inline void load_a(AStep<MT, MODE> &x, const AOpL<TA> &a, int s)
     const int o = (s - a.s0) * 2 * kStep;
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
-        x.a0[mt] = *(const half8 *)(a.q + a.qoff[mt] + o);
-        x.a1[mt] = *(const half8 *)(a.q + a.qoff[mt] + o + 16);
+        x.raw[2 * mt] = *(const u32x4 *)(a.q + a.qoff[mt] + o);
+        x.raw[2 * mt + 1] = *(const u32x4 *)(a.q + a.qoff[mt] + o + 16);
     }
     if (MODE == kStepDs) {
 #pragma unroll
@@ -524,56 +589,50 @@ __device__ inline void load_a(AStep<MT, MODE> &x, const AOpL<TA> &a, int s)
 }
 
 template <int MT, int MODE, int TA>
-__device__ inline void load_a(AStep<MT, MODE> &x, const AOp<TA> &a, int s)
+__device__ inline void publish_a(const AStep<MT, MODE> &, const AOpL<TA> &)
+{
+}
+
+template <int MT, int MODE, int TA>
+__device__ inline void operand_a(half8 *av, const AStep<MT, MODE> &x, const AOpL<TA> &, int j)
 {
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        x.a0[mt] = as_h8(__builtin_amdgcn_raw_buffer_load_b128(a.q, a.qoff[mt], s * 2 * kStep, 0));
-        x.a1[mt] = as_h8(__builtin_amdgcn_raw_buffer_load_b128(a.q, a.qoff[mt], s * 2 * kStep + 16, 0));
-    }
-    if (MODE == kStepDs) {
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(a.ds, a.doff[mt], s * a.ld4, 0);
-            __builtin_memcpy(&x.dv[mt], &v, 16);
-        }
-    }
+    for (int mt = 0; mt < MT; mt++) av[mt] = as_h8(x.raw[2 * mt + j]);
 }
 
 // acc[mt][t][i] += the step's contribution.
 // s: the step's number within its scale unit.
-template <class D, int MT, int MODE, int s>
-__device__ inline void mm_step(const typename D::Raw &w, typename D::State &st, const AStep<MT, MODE> &x, int lane,
-                               f32x4 (*acc)[4])
+template <class D, int MT, int MODE, int s, class AS>
+__device__ inline void mm_step(const typename D::Raw &w, typename D::State &st, const AStep<MT, MODE> &x, const AS &A,
+                               int lane, f32x4 (*acc)[4])
 {
     const half8 ones = (half8)(half_t)1.0f;
     const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     D::begin(w, st, s);
-    f32x4 sum[MT][2];
-    if (D::kMin) {
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            sum[mt][0] = mfma(x.a0[mt], ones, zero);
-            sum[mt][1] = mfma(x.a1[mt], ones, zero);
+    for (int j = 0; j < 2; j++) {
+        half8 av[MT];
+        operand_a(av, x, A, j);
+        f32x4 sum[MT];
+        if (D::kMin) {
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) sum[mt] = mfma(av[mt], ones, zero);
         }
-    }
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
+        for (int t = 0; t < 4; t++) {
             half8 b;
             float d, mn;
             D::operand(w, st, s, lane, t, j, b, d, mn);
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) {
-                const f32x4 r = mfma(j ? x.a1[mt] : x.a0[mt], b, zero);
+                const f32x4 r = mfma(av[mt], b, zero);
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     if (MODE == kRow) {
                         acc[mt][t][i] = __builtin_fmaf(d, r[i], acc[mt][t][i]);
-                        if (D::kMin) acc[mt][t][i] = __builtin_fmaf(-mn, sum[mt][j][i], acc[mt][t][i]);
+                        if (D::kMin) acc[mt][t][i] = __builtin_fmaf(-mn, sum[mt][i], acc[mt][t][i]);
                     } else {
-                        const float v = D::kMin ? d * r[i] - mn * sum[mt][j][i] : d * r[i];
+                        const float v = D::kMin ? d * r[i] - mn * sum[mt][i] : d * r[i];
                         acc[mt][t][i] = __builtin_fmaf(x.dv[mt][i], v, acc[mt][t][i]);
                     }
                 }
@@ -611,6 +670,7 @@ __device__ inline void mm_steps(const Planes &W, int rb, int s0, int s1, int lan
     AStep<MT, MODE> x0, x1;
     load_a(x0, A, s0);
     D::template load<true>(w0, W, rb, s0, lane);
+    publish_a(x0, A);
     // One step: the next step's loads, then this one's products.  k: the step's
     // number modulo the loop's unroll, so a super-block decoder knows at compile time
     // which steps start a scale unit (a share starts and ends on whole units): its
@@ -622,8 +682,9 @@ __device__ inline void mm_steps(const Planes &W, int rb, int s0, int s1, int lan
         load_a(xn, A, min(s + 1, sl));
         D::template load<(k + 1) % D::kSpu == 0>(wn, W, rb, ws(s + 1), lane);
         __builtin_amdgcn_sched_barrier(0);
-        mm_step<D, MT, MODE, k % D::kSpu>(wc, st, xc, lane, acc);
+        mm_step<D, MT, MODE, k % D::kSpu>(wc, st, xc, A, lane, acc);
         __builtin_amdgcn_sched_barrier(0);
+        publish_a(xn, A);
     };
     using C0 = std::integral_constant<int, 0>;
     using C1 = std::integral_constant<int, 1>;
@@ -643,7 +704,7 @@ __device__ inline void mm_steps(const Planes &W, int rb, int s0, int s1, int lan
             step(C0{}, w0, w1, x0, x1, s);
             step(C0{}, w1, w0, x1, x0, s + 1);
         }
-        if (s < s1) mm_step<D, MT, MODE, 0>(w0, st, x0, lane, acc);
+        if (s < s1) mm_step<D, MT, MODE, 0>(w0, st, x0, A, lane, acc);
     }
 }
 
@@ -694,10 +755,12 @@ __device__ inline bool chunk_of(const Dispatch &d, int ci, int &e, int &p0, int 
 // 64-row block, K share), chunks fastest.  Wave w: matrix w >> 1 (gate, up), half w & 1 of
 // the workgroup's K units; the four are summed through LDS and wave 0 applies
 // SiLU(g) * u to its 64 rows x 16 MT tokens.
-template <class D, int MT>
+template <class D, int MT, bool kStage>
 __global__ __launch_bounds__(256) MM_ATTR void k_mm_gateup(MmArgs a)
 {
+    // the wavefronts' staged activations in the K loop, the gate/up exchange after it
     __shared__ f32x4 xch[3][MT][4][64];
+    static_assert(sizeof xch >= 4 * MT * kStageBytes, "the staged activations fit the exchange's LDS");
     int e, p0, nt;
     if (!chunk_of<MT>(a.d, (int)(blockIdx.x % a.nchunk), e, p0, nt)) return;  // uniform over the workgroup
     const int rbk = (int)(blockIdx.x / a.nchunk), rb = rbk / a.KS, ks = rbk % a.KS;
@@ -708,18 +771,23 @@ __global__ __launch_bounds__(256) MM_ATTR void k_mm_gateup(MmArgs a)
     const int ub = u0 + half * hu, ue = min(u0 + upw, ub + hu);
     const Planes W = planes(mat ? a.w1 : a.w0, e);
     const int n = lane & 15, gq = lane >> 4;
-    AOp<MT> A;
+    AOp<MT, kStage> A;
     A.q = make_rsrc(a.x.q, (size_t)a.x.ld * a.H * 2);  // x: ld = tokens
     A.ds = make_rsrc(a.x.ds, (size_t)(a.H / kStep) * a.x.ld * 4);
     A.ld4 = a.x.ld * 4;
     float dvr[MT][4];  // x's per-row descales of the lane's result tokens
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
-        A.qoff[mt] = a.d.rows[p0 + min(16 * mt + n, nt - 1)] * a.H * 2 + 32 * gq;
         A.doff[mt] = 0;
 #pragma unroll
         for (int i = 0; i < 4; i++) dvr[mt][i] = a.x.ds[a.d.rows[p0 + min(16 * mt + 4 * gq + i, nt - 1)]];
     }
+#pragma unroll
+    for (int i = 0; i < 2 * MT; i++) {
+        if constexpr (kStage) A.qoff[i] = a.d.rows[p0 + min(8 * i + (lane >> 3), nt - 1)] * a.H * 2 + 16 * (lane & 7);
+        else A.qoff[i] = a.d.rows[p0 + min(8 * (i & ~1) + n, nt - 1)] * a.H * 2 + 32 * gq;
+    }
+    if constexpr (kStage) A.stage_at((char *)xch + wv * MT * kStageBytes, lane);
     f32x4 acc[MT][4];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
@@ -732,6 +800,7 @@ __global__ __launch_bounds__(256) MM_ATTR void k_mm_gateup(MmArgs a)
         for (int t = 0; t < 4; t++)
 #pragma unroll
             for (int i = 0; i < 4; i++) acc[mt][t][i] *= dvr[mt][i];
+    if constexpr (kStage) __syncthreads();  // every wavefront's last operand reads are done
     if (wv) {
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
@@ -817,12 +886,12 @@ __global__ __launch_bounds__(256) void k_act_reduce(MmArgs a)
 // the last position, out-of-range zero) activations and are not stored.  Position
 // p's result goes to row rows[p] * kk + slots[p] of the output.
 //
-// kPart: gate/up split its K over KSg workgroups and left the partials in `part`.
+// kAPart: gate/up split its K over KSg workgroups and left the partials in `part`.
 // The workgroup finishes the activations it reads itself, k_act_reduce's sums in
 // the same order (so the same bits), for its chunk's tokens and its K range only,
 // into LDS (dynamic: 16 MT rows of its steps, and their descales); the K loop then
 // reads them from there.  No launch between gate/up and down.
-template <class D, int MT, bool kPart>
+template <class D, int MT, ASource kSrc>
 __global__ __launch_bounds__(256) MM_ATTR void k_mm_down(MmArgs a)
 {
     int e, p0, nt;
@@ -846,7 +915,7 @@ __global__ __launch_bounds__(256) MM_ATTR void k_mm_down(MmArgs a)
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int t = 0; t < 4; t++) acc[mt][t] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-    if constexpr (kPart) {
+    if constexpr (kSrc == kAPart) {
         extern __shared__ __attribute__((aligned(16))) char lds_act[];
         const int sw = upw * D::kSpu, s0 = u0 * D::kSpu;  // the workgroup's steps
         const int rowb = sw * 2 * kStep;
@@ -902,14 +971,21 @@ __global__ __launch_bounds__(256) MM_ATTR void k_mm_down(MmArgs a)
         mm_live<D, MT, kStepDs>(W, rb, s0, s0 + sw, lane, A, acc, nt);
     } else {
         if (rb >= a.H / kRowBlock) return;  // no barriers in this kernel
-        AOp<MT> A;
+        constexpr bool kStage = kSrc == kAStaged;
+        AOp<MT, kStage> A;
         A.q = make_rsrc(a.x.q, (size_t)a.P * a.I * 2);
         A.ds = make_rsrc(a.x.ds, (size_t)(a.I / kStep) * a.x.ld * 4);
         A.ld4 = a.x.ld * 4;
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            A.qoff[mt] = (p0 + 16 * mt + n) * a.I * 2 + 32 * gq;
-            A.doff[mt] = (p0 + 16 * mt + 4 * gq) * 4;
+        for (int mt = 0; mt < MT; mt++) A.doff[mt] = (p0 + 16 * mt + 4 * gq) * 4;
+#pragma unroll
+        for (int i = 0; i < 2 * MT; i++) {
+            if constexpr (kStage) A.qoff[i] = (p0 + 8 * i + (lane >> 3)) * a.I * 2 + 16 * (lane & 7);
+            else A.qoff[i] = (p0 + 8 * (i & ~1) + n) * a.I * 2 + 32 * gq;
+        }
+        if constexpr (kStage) {
+            __shared__ __attribute__((aligned(16))) char ast[4 * MT * kStageBytes];
+            A.stage_at(ast + wv * MT * kStageBytes, lane);
         }
         mm_live<D, MT, kStepDs>(W, rb, u0 * D::kSpu, (u0 + upw) * D::kSpu, lane, A, acc, nt);
     }
@@ -1068,7 +1144,7 @@ __global__ __launch_bounds__(256) void k_combine_rows(const float *__restrict__ 
 
 static int steps_per_unit(int type) { return tile_fmt(type).spu; }
 
-// Dynamic LDS of a kPart down workgroup: 16 rows of its steps in the activation
+// Dynamic LDS of a kAPart down workgroup: 16 rows of its steps in the activation
 // format, and a descale per (step, row).
 constexpr size_t kFuseLdsMax = 64 * 1024;
 static size_t down_part_lds(int down_type, int I, int ks_dn, int mt)
@@ -1138,6 +1214,7 @@ MmPlan plan_mm(int gate_type, int down_type, int H, int I, int P, int max_u, int
     } else {
         p.kind = kMmDecode;
         p.mt = mean >= kWideMean ? 2 : 1;
+        p.stage = mean >= kStageMean;
     }
     p.chunk = 16 * p.mt;
     p.nchunk = P / p.chunk + max_u;
@@ -1153,7 +1230,7 @@ MmPlan plan_mm(int gate_type, int down_type, int H, int I, int P, int max_u, int
 #ifdef ANEDVD_KS_DN
     if (max_u > 64 && (I / kStep / steps_per_unit(down_type)) % ANEDVD_KS_DN == 0) p.ks_dn = ANEDVD_KS_DN;
 #endif
-    // A K-split gate/up is finished inside the down kernel (k_mm_down<kPart>) when
+    // A K-split gate/up is finished inside the down kernel (k_mm_down<kAPart>) when
     // a down workgroup's rows of its K range fit the LDS budget and its prologue
     // has at most 64 (token, step) pieces, four memory round trips (16 pieces each),
     // even if every token of the call sends a slot to the same expert (a chunk
@@ -1165,39 +1242,38 @@ MmPlan plan_mm(int gate_type, int down_type, int H, int I, int P, int max_u, int
 
 // ------------------------------------------------------------- launchers
 
-template <class D, int MT>
+template <class D, int MT, bool kStage>
 static int launch_gateup_t(const MmArgs &a, hipStream_t st)
 {
     const size_t wgs = (size_t)a.nchunk * (a.I / kRowBlock) * a.KS;
-    hipLaunchKernelGGL((k_mm_gateup<D, MT>), dim3((unsigned)wgs), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_mm_gateup<D, MT, kStage>), dim3((unsigned)wgs), dim3(256), 0, st, a);
     ANEDVD_HIP(hipGetLastError());
     return ANEDVD_OK;
 }
 
-template <class D, int MT>
+template <class D, int MT, ASource kSrc>
 static int launch_down_t(const MmArgs &a, hipStream_t st)
 {
     const size_t wgs = (size_t)a.nchunk * ((a.H / kRowBlock + kWaves - 1) / kWaves) * a.KS;
-    if (a.KSg > 1) {
-        const size_t lds = down_part_lds(a.w0.type, a.I, a.KS, MT);
-        hipLaunchKernelGGL((k_mm_down<D, MT, true>), dim3((unsigned)wgs), dim3(256), lds, st, a);
-    } else {
-        hipLaunchKernelGGL((k_mm_down<D, MT, false>), dim3((unsigned)wgs), dim3(256), 0, st, a);
-    }
+    const size_t lds = kSrc == kAPart ? down_part_lds(a.w0.type, a.I, a.KS, MT) : 0;
+    hipLaunchKernelGGL((k_mm_down<D, MT, kSrc>), dim3((unsigned)wgs), dim3(256), lds, st, a);
     ANEDVD_HIP(hipGetLastError());
     return ANEDVD_OK;
 }
 
 template <class D>
-static int launch_gateup_d(const MmArgs &a, int mt, hipStream_t st)
+static int launch_gateup_d(const MmArgs &a, const MmPlan &p, hipStream_t st)
 {
-    return mt == 2 ? launch_gateup_t<D, 2>(a, st) : launch_gateup_t<D, 1>(a, st);
+    if (p.mt == 2) return launch_gateup_t<D, 2, true>(a, st);
+    return p.stage ? launch_gateup_t<D, 1, true>(a, st) : launch_gateup_t<D, 1, false>(a, st);
 }
 
 template <class D>
-static int launch_down_d(const MmArgs &a, int mt, hipStream_t st)
+static int launch_down_d(const MmArgs &a, const MmPlan &p, hipStream_t st)
 {
-    return mt == 2 ? launch_down_t<D, 2>(a, st) : launch_down_t<D, 1>(a, st);
+    if (a.KSg > 1) return p.mt == 2 ? launch_down_t<D, 2, kAPart>(a, st) : launch_down_t<D, 1, kAPart>(a, st);
+    if (p.mt == 2) return launch_down_t<D, 2, kAStaged>(a, st);
+    return p.stage ? launch_down_t<D, 1, kAStaged>(a, st) : launch_down_t<D, 1, kASelf>(a, st);
 }
 
 int launch_expert_gateup(const QMat &gate, const QMat &up, const ActQ &x, int H, int I, const Dispatch &d, int P,
@@ -1226,17 +1302,17 @@ int launch_expert_gateup(const QMat &gate, const QMat &up, const ActQ &x, int H,
     int rc;
     switch (gate.type) {
     case ANEDVD_Q8_0:
-    case ANEDVD_Q8_1: rc = launch_gateup_d<MQ8_0>(a, plan.mt, st); break;  // one tile layout
-    case ANEDVD_F16: rc = launch_gateup_d<MF16>(a, plan.mt, st); break;
-    case ANEDVD_Q4_0: rc = launch_gateup_d<MQ4_0>(a, plan.mt, st); break;
-    case ANEDVD_Q4_1: rc = launch_gateup_d<MQ4_1>(a, plan.mt, st); break;
-    case ANEDVD_Q5_0: rc = launch_gateup_d<MQ5_0>(a, plan.mt, st); break;
-    case ANEDVD_Q5_1: rc = launch_gateup_d<MQ5_1>(a, plan.mt, st); break;
-    case ANEDVD_Q2_K: rc = launch_gateup_d<MQ2_K>(a, plan.mt, st); break;
-    case ANEDVD_Q3_K: rc = launch_gateup_d<MQ3_K>(a, plan.mt, st); break;
-    case ANEDVD_Q4_K: rc = launch_gateup_d<MQ4_K>(a, plan.mt, st); break;
-    case ANEDVD_Q5_K: rc = launch_gateup_d<MQ5_K>(a, plan.mt, st); break;
-    case ANEDVD_Q6_K: rc = launch_gateup_d<MQ6_K>(a, plan.mt, st); break;
+    case ANEDVD_Q8_1: rc = launch_gateup_d<MQ8_0>(a, plan, st); break;  // one tile layout
+    case ANEDVD_F16: rc = launch_gateup_d<MF16>(a, plan, st); break;
+    case ANEDVD_Q4_0: rc = launch_gateup_d<MQ4_0>(a, plan, st); break;
+    case ANEDVD_Q4_1: rc = launch_gateup_d<MQ4_1>(a, plan, st); break;
+    case ANEDVD_Q5_0: rc = launch_gateup_d<MQ5_0>(a, plan, st); break;
+    case ANEDVD_Q5_1: rc = launch_gateup_d<MQ5_1>(a, plan, st); break;
+    case ANEDVD_Q2_K: rc = launch_gateup_d<MQ2_K>(a, plan, st); break;
+    case ANEDVD_Q3_K: rc = launch_gateup_d<MQ3_K>(a, plan, st); break;
+    case ANEDVD_Q4_K: rc = launch_gateup_d<MQ4_K>(a, plan, st); break;
+    case ANEDVD_Q5_K: rc = launch_gateup_d<MQ5_K>(a, plan, st); break;
+    case ANEDVD_Q6_K: rc = launch_gateup_d<MQ6_K>(a, plan, st); break;
     default:
         set_error("expert gate/up: ggml type %d has no kernel", gate.type);
         return ANEDVD_E_UNSUPPORTED_TYPE;
@@ -1277,17 +1353,17 @@ int launch_expert_down(const QMat &down, const ActQ &act, int H, int I, const Di
     }
     switch (down.type) {
     case ANEDVD_Q8_0:
-    case ANEDVD_Q8_1: return launch_down_d<MQ8_0>(a, plan.mt, st);
-    case ANEDVD_F16: return launch_down_d<MF16>(a, plan.mt, st);
-    case ANEDVD_Q4_0: return launch_down_d<MQ4_0>(a, plan.mt, st);
-    case ANEDVD_Q4_1: return launch_down_d<MQ4_1>(a, plan.mt, st);
-    case ANEDVD_Q5_0: return launch_down_d<MQ5_0>(a, plan.mt, st);
-    case ANEDVD_Q5_1: return launch_down_d<MQ5_1>(a, plan.mt, st);
-    case ANEDVD_Q2_K: return launch_down_d<MQ2_K>(a, plan.mt, st);
-    case ANEDVD_Q3_K: return launch_down_d<MQ3_K>(a, plan.mt, st);
-    case ANEDVD_Q4_K: return launch_down_d<MQ4_K>(a, plan.mt, st);
-    case ANEDVD_Q5_K: return launch_down_d<MQ5_K>(a, plan.mt, st);
-    case ANEDVD_Q6_K: return launch_down_d<MQ6_K>(a, plan.mt, st);
+    case ANEDVD_Q8_1: return launch_down_d<MQ8_0>(a, plan, st);
+    case ANEDVD_F16: return launch_down_d<MF16>(a, plan, st);
+    case ANEDVD_Q4_0: return launch_down_d<MQ4_0>(a, plan, st);
+    case ANEDVD_Q4_1: return launch_down_d<MQ4_1>(a, plan, st);
+    case ANEDVD_Q5_0: return launch_down_d<MQ5_0>(a, plan, st);
+    case ANEDVD_Q5_1: return launch_down_d<MQ5_1>(a, plan, st);
+    case ANEDVD_Q2_K: return launch_down_d<MQ2_K>(a, plan, st);
+    case ANEDVD_Q3_K: return launch_down_d<MQ3_K>(a, plan, st);
+    case ANEDVD_Q4_K: return launch_down_d<MQ4_K>(a, plan, st);
+    case ANEDVD_Q5_K: return launch_down_d<MQ5_K>(a, plan, st);
+    case ANEDVD_Q6_K: return launch_down_d<MQ6_K>(a, plan, st);
     default:
         set_error("expert down: ggml type %d has no kernel", down.type);
         return ANEDVD_E_UNSUPPORTED_TYPE;

@@ -106,6 +106,7 @@ struct MmPlan {
     int small;    // grouped GEMM: groups of at most this many tokens run on one 16-token tile each (0 = none)
     int nsmall;   // grouped GEMM with small: capacity of the small groups' list (max_u)
     int xper;     // grouped GEMM with contig: chunks per XCD range of the work list (0 = none)
+    int stage;    // decode: activations read row by row and staged in LDS
     int fuse;     // decode, ks_gu > 1: the down kernel finishes gate/up's K partials (no k_act_reduce)
 };
 bool mm_supported(int type);
