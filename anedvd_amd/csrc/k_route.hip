@@ -230,6 +230,78 @@ __global__ __launch_bounds__(256) void k_router(const float *__restrict__ wt, co
     }
 }
 
+// The same logits, one wavefront per (8 experts, token), for calls of a few tokens: lane
+// 8 g + l runs chain l of expert 8 blockIdx.x + g with kAhead 8-j blocks of weights in
+// flight.  The call is bound by the latency of its weight loads and by what one CU
+// streams: k_router's 32-expert blocks read 256 KB each (Qwen3) two blocks ahead, the
+// fused routing workgroup the whole megabyte.  Here 16 CUs read 64 KB each.  Routing
+// stage with a cold router, k_router or fused / this kernel (us): Qwen3 1 token 21.4 /
+// 14.9, 7 tokens 17.4 / 15.0, 16 tokens 17.3 / 16.2; DeepSeek-V2-Lite 4 tokens 15.2 /
+// 13.5, 32 tokens 17.0 / 16.0.
+__global__ __launch_bounds__(64) void k_router_wave(const float *__restrict__ wt, const uint16_t *__restrict__ w,
+                                                    const float *__restrict__ x, int E, int H,
+                                                    float *__restrict__ logits)
+{
+    constexpr int kAhead = 8;
+    extern __shared__ float xs[];  // [8][JP]
+    const int J = H >> 3, H8 = J * 8, JP = router_stride(J), NB = (int)router_blocks(H), NBF = J / 8;
+    const int e0 = blockIdx.x * 8, lane = threadIdx.x, l = lane & 7;
+    const float *xt = x + (size_t)blockIdx.y * H;
+    // the block's experts: layout group e0 / 64, from expert e0 % 64 of it
+    const rsrc_t rs = make_rsrc(wt + ((size_t)(e0 / kRouterGroup) * NB * kRouterGroup + e0 % kRouterGroup) * 64,
+                                (size_t)NB * kRouterGroup * 256);
+    float4 wb[kAhead][2];
+    auto load = [&](int k, int jb) {  // past the last block: outside the descriptor's range, 0 without a request
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            wb[k][h] = __builtin_bit_cast(
+                float4, __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 32 + 16 * h, jb * kRouterGroup * 256, 0));
+    };
+#pragma unroll
+    for (int k = 0; k < kAhead; k++) load(k, k);
+    constexpr int kB = 8;  // staging loads in flight per lane
+    for (int i0 = lane; i0 < H8; i0 += kB * 64) {
+        float v[kB];
+#pragma unroll
+        for (int b = 0; b < kB; b++) v[b] = i0 + 64 * b < H8 ? xt[i0 + 64 * b] : 0.0f;
+#pragma unroll
+        for (int b = 0; b < kB; b++) {
+            const int i = i0 + 64 * b;
+            if (i < H8) xs[(i & 7) * JP + (i >> 3)] = v[b];
+        }
+    }
+    __syncthreads();
+    float acc = 0.0f;
+    auto add = [&](int k, int jb, int nq) {
+        const float wf[8] = {wb[k][0].x, wb[k][0].y, wb[k][0].z, wb[k][0].w,
+                             wb[k][1].x, wb[k][1].y, wb[k][1].z, wb[k][1].w};
+        const float *xr = &xs[l * JP + 8 * jb];
+#pragma unroll
+        for (int q = 0; q < 8; q++)
+            if (q < nq) acc = __fadd_rn(acc, __fmul_rn(xr[q], wf[q]));
+    };
+    int jb = 0;
+    for (; jb + kAhead <= NBF; jb += kAhead) {
+#pragma unroll
+        for (int k = 0; k < kAhead; k++) {
+            add(k, jb + k, 8);
+            load(k, jb + k + kAhead);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kAhead; k++)
+        if (jb + k < NB) add(k, jb + k, min(8, J - 8 * (jb + k)));
+    // ordered sum of the chains, then the scalar tail
+    float sum = __shfl(acc, lane & ~7, 64);
+    for (int q = 1; q < 8; q++) sum = __fadd_rn(sum, __shfl(acc, (lane & ~7) + q, 64));
+    const int e = e0 + (lane >> 3);
+    if (e < E && l == 0) {
+        const uint16_t *row = w + (size_t)e * H;
+        for (int i = H8; i < H; i++) sum = __fadd_rn(sum, __fmul_rn(f16_bits_to_f32(row[i]), xt[i]));
+        logits[(size_t)blockIdx.y * E + e] = sum;
+    }
+}
+
 int launch_router_layout(const uint16_t *d_w, int E, int H, float *d_wt, hipStream_t st)
 {
     const size_t n = router_layout_floats(E, H);
@@ -247,12 +319,22 @@ int launch_router(const float *d_wt, const uint16_t *d_w, const float *d_x, int 
         set_error("router: hidden size %d too large", H);
         return ANEDVD_E_INVALID_ARG;
     }
-    // Two tokens and two experts per lane once the grid still has about two
-    // wavefronts per SIMD that way (Qwen3 512 tokens, DeepSeek-V2-Lite 1024: 11.5
-    // and 11.8 us against 13.1 and 13.4 at one expert, 19.9 and 20.6 at one token
-    // and one expert); one of each below (64 tokens of 128 experts: 5.1 against
+    // Two tokens and two experts per lane once the grid still has about one
+    // wavefront per SIMD that way (Qwen3 333 tokens 11.4 against 14.9 us at one and one,
+    // 256 tokens 10.6 / 10.8, 192 tokens 10.7 / 8.9, DeepSeek-V2-Lite 768 tokens 11.8 /
+    // 15.4; Qwen3 512 tokens and DeepSeek-V2-Lite 1024 11.5 and 11.8 us against 13.1 and
+    // 13.4 at one expert); one of each below (64 tokens of 128 experts: 5.1 against
     // 6.3 us at two tokens), and one expert for E < 64 (Mixtral's E = 8).
-    const bool big = E >= 64 && (long)T * E >= 65536;
+    const bool big = E >= 64 && (long)T * E >= 32768;
+    // A few tokens: one wavefront per 8 experts and token (up to 2048 (token, expert)
+    // pairs; 32 tokens of 128 experts: 17.1 against 17.9 us).
+    const size_t wave_lds = (size_t)8 * router_stride(H >> 3) * 4;
+    if (T <= 64 && (long)T * E <= 2048 && wave_lds <= 65536) {
+        hipLaunchKernelGGL(k_router_wave, dim3((unsigned)((E + 7) / 8), (unsigned)T), dim3(64), wave_lds, st, d_wt, d_w,
+                           d_x, E, H, d_logits);
+        ANEDVD_HIP(hipGetLastError());
+        return ANEDVD_OK;
+    }
     auto go = [&](auto tt, auto ex) -> int {
         constexpr int TT = decltype(tt)::value, EX = decltype(ex)::value;
         const size_t lds = (size_t)TT * 8 * router_stride(H >> 3) * 4;
@@ -1175,9 +1257,15 @@ bool route_fusable(int T, int)
     return T > 0 && T <= kFusedTokens;
 }
 
+// The largest router (as f32) the routing workgroup reads itself: one CU streams it
+// all.  Mixtral's 128 KB 12.6 us fused against 15.7 us in a launch of its own;
+// DeepSeek-V2-Lite's 512 KB: a one-token layer 33.4 / 33.9 us; Qwen3's 1 MB 21.4 / 14.9 us.
+constexpr size_t kFusedRouterBytes = 512 * 1024;
+
 bool route_router_fusable(int T, int E, int H)
 {
     return route_fusable(T, E) && T * E * 8 <= kDispThreads && E <= kMaxExperts &&
+           (size_t)E * H * 4 <= kFusedRouterBytes &&
            (size_t)T * 8 * router_stride(H >> 3) * 4 <= sizeof(DispLds);
 }
 

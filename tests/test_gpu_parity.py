@@ -91,7 +91,7 @@ def test_resident_experts_bit_exact(ctx, types):
                                               (100, 1003, 5), (8, 64, 70000), (256, 1024, 300)])
 def test_matmul_f16_bit_exact(ctx, out_dim, in_dim, n):
     """The router GEMV (cpu.matmulF16's chains) at the shapes of both launch forms:
-    a token and an expert per lane, and two of each (>= 64 experts and >= 65536
+    a token and an expert per lane, and two of each (>= 64 experts and >= 32768
     token-expert pairs: (64, 2048, 1024), (128, 2048, 512), and (100, 1003, 700) with
     a partial second expert half and a partial last 8-j block plus a scalar tail; an
     odd token count, whose last workgroup has one token), a hidden size below one
@@ -100,6 +100,21 @@ def test_matmul_f16_bit_exact(ctx, out_dim, in_dim, n):
     1024, 300)."""
     w = (synth.normal(1, out_dim, out_dim * in_dim) * 0.02).astype(np.float16).reshape(out_dim, in_dim)
     x = synth.normal(2, in_dim, n * in_dim).astype(np.float32).reshape(n, in_dim)
+    got = ctx.matmul_f16(w, x)
+    want = np.stack([O.matmul_f16(w, x[i]) for i in range(n)])
+    assert np.array_equal(bits(got), bits(want))
+
+
+@pytest.mark.parametrize("E,H,n", [(128, 2048, 16), (128, 2048, 17), (64, 2048, 32), (9, 1003, 64), (8, 4096, 64),
+                                   (8, 4096, 65), (13, 520, 1), (256, 512, 8), (70, 576, 3), (1, 7, 2), (72, 64, 5),
+                                   (128, 2048, 255), (128, 2048, 256)])
+def test_matmul_f16_few_tokens_bit_exact(ctx, E, H, n):
+    """The router GEMV's one wavefront per (8 experts, token) up to 2048 (token, expert)
+    pairs and 64 tokens, and both sides of that line and of the two-by-two kernel's
+    (32768 pairs): whole and partial runs of eight 8-j blocks, a scalar tail, experts
+    that end inside a wavefront and inside a 64-expert group."""
+    w = (synth.normal(3, E, E * H) * 0.02).astype(np.float16).reshape(E, H)
+    x = synth.normal(4, H, n * H).astype(np.float32).reshape(n, H)
     got = ctx.matmul_f16(w, x)
     want = np.stack([O.matmul_f16(w, x[i]) for i in range(n)])
     assert np.array_equal(bits(got), bits(want))
