@@ -70,6 +70,12 @@ constexpr int kWaves = 4;
 // mean 25 368 / 281.  (64-token chunks: Qwen3 Q8_0 mean 21 186, the accumulators and
 // activations then leave one or two wavefronts per SIMD.)
 constexpr int kWideMean = 10;
+// ... and the gate and up weights they read at least: below, a second pass over an
+// expert hits the L2s and half the workgroups only cost parallelism (the tiny layer,
+// 9 MB, 64 tokens 26.2 us at 16-token chunks, 28.2 at 32; the generic f16 layer with
+// its 3 MB shared expert, 34 tokens 66 and 68 us, while its 34 MB of routed experts at
+// 64 tokens take 77 and 70.5 us).
+constexpr size_t kWideBytes = (size_t)16 << 20;
 // Mean group size from which the decode kernels stage their activations (ASource):
 // with fewer tokens per group a direct load touches few lines anyway.
 constexpr int kStageMean = 2;
@@ -1213,7 +1219,8 @@ MmPlan plan_mm(int gate_type, int down_type, int H, int I, int P, int max_u, int
         p.nsmall = p.small ? max_u : 0;
     } else {
         p.kind = kMmDecode;
-        p.mt = mean >= kWideMean ? 2 : 1;
+        const size_t gu_bytes = (size_t)max_u * I * H / block_elems(gate_type) * block_bytes(gate_type) * 2;
+        p.mt = mean >= kWideMean && gu_bytes >= kWideBytes ? 2 : 1;
         p.stage = mean >= kStageMean;
     }
     p.chunk = 16 * p.mt;

@@ -442,12 +442,12 @@ def test_forward_grouped_every_live_tile_count(ctx, types):
     assert st["chunk"] == (128 if wide_gu or wide_dn else 64)  # gate/up and down pick their widths apart
 
 
-@pytest.mark.parametrize("shape", [(1024, 512), (256, 8192)], ids=["k-split", "whole-k"])
-@pytest.mark.parametrize("types", FORMATS, ids=lambda t: "/".join(W.TYPE_NAMES[x] for x in t))
+@pytest.mark.parametrize("types,shape", [(t, (2048, 2048)) for t in FORMATS] + [(t, (512, 8192)) for t in FORMATS[:3]],
+                         ids=lambda v: "/".join(W.TYPE_NAMES[x] for x in v) if len(v) == 3 else f"h{v[0]}-i{v[1]}")
 def test_forward_decode_32_token_chunks(ctx, types, shape):
-    """The decode kernels' 32-token chunks (mean group 18): groups at the edges of one
-    and two 16-token tiles and of a second chunk, with gate/up's K split (finished in
-    the down kernel) and whole."""
+    """The decode kernels' 32-token chunks (mean group 18, gate and up of 16 MB and
+    more): groups at the edges of one and two 16-token tiles and of a second chunk, with
+    gate/up's K split (finished in the down kernel) and whole."""
     sizes = [1, 15, 16, 17, 31, 32, 33, 3]
     lg = _logits_for_groups(sizes, seed=31)
     spec = dataclasses.replace(W.MIXTRAL_8X7B_Q4_0, name="mm-32", hidden=shape[0], inter=shape[1],
