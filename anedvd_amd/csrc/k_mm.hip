@@ -10,10 +10,11 @@
 // owns 64 weight rows (four 16-row tiles) and streams their K span in steps of 64
 // columns, one global load per lane per tile per step.  Each lane turns its 16
 // quants into the f16 B operands of two v_mfma_f32_16x16x32_f16 (byte permutes
-// under the exponent byte 0x64 give 1024 + q exactly); the A operand is 16 tokens
-// of the group (padded by repeating the last token), read straight from the
-// L2-resident activations, so the weights are read once per 16 tokens and no
-// LDS staging or barrier sits in the stream.  Each MFMA covers one 32-column
+// under the exponent byte 0x64 give 1024 + q exactly); the A operands are one or two
+// tiles of 16 tokens of the group (padded by repeating the last token), read from the
+// L2-resident activations (row by row through the wavefront's own LDS where groups hold
+// several tokens), so the weights are read once per 16 or 32 tokens and no barrier sits
+// in the stream.  Each MFMA covers one 32-column
 // block of one 16-row tile, so the block's scale (and Q4_K's min term, with the
 // block sums of the activations from an MFMA against ones) is applied to its
 // f32 result together with the activations' per-64-column descale.  Q6_K's

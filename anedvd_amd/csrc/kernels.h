@@ -79,7 +79,7 @@ int launch_dispatch(const uint32_t *d_idx, int T, int k, int E, const Dispatch &
 // one-workgroup dispatch launch.
 bool route_fusable(int T, int E);
 // route_router_fusable(T, E, H): the fused launch can also form the router logits
-// (a chain per thread); then d_logits is null and d_rwt / d_rw the router (in
+// (a chain per thread, the router small enough for one CU); then d_logits is null and d_rwt / d_rw the router (in
 // launch_router_layout's layout, as stored), and d_x the call's activations.
 bool route_router_fusable(int T, int E, int H);
 int launch_route_and_dispatch(const float *d_logits, int T, int E, int k, int norm, float *d_probs, uint32_t *d_idx,
