@@ -549,18 +549,28 @@ __device__ inline void load_a(AStep<MT, MODE> &x, const AOp<TA, kStage> &a, int 
     }
 }
 
-// Puts a loaded step where the operands are read from (the step before it is done).
+// Puts a loaded step where the operands are read from.  The lanes read each other's
+// pieces: the hardware does one wavefront's LDS accesses in order, and the fences here
+// and before the step's first operand read hold the compiler to that order.  (They cost
+// no instruction or register there; right after the stores the second one also pinned
+// the next step's loads: Q4_0 gate/up 80 -> 84 VGPRs, 64 tokens of 64 experts 63.2 ->
+// 65.2 us.)
+__device__ inline void stage_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); }
+
 template <int MT, int MODE, int TA, bool kStage>
 __device__ inline void publish_a(const AStep<MT, MODE> &x, const AOp<TA, kStage> &a)
 {
-    if constexpr (!kStage) return;
+    if constexpr (kStage) {
+        stage_fence();
 #pragma unroll
-    for (int i = 0; i < 2 * MT; i++) *(u32x4 *)(a.st + 1024 * i + ((i & 1) ? a.wr ^ 16 : a.wr)) = x.raw[i];
+        for (int i = 0; i < 2 * MT; i++) *(u32x4 *)(a.st + 1024 * i + ((i & 1) ? a.wr ^ 16 : a.wr)) = x.raw[i];
+    }
 }
 
 template <int MT, int MODE, int TA, bool kStage>
 __device__ inline void operand_a(half8 *av, const AStep<MT, MODE> &x, const AOp<TA, kStage> &a, int j)
 {
+    if (kStage && j == 0) stage_fence();
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
         if constexpr (kStage) av[mt] = *(const half8 *)(a.st + kStageBytes * mt + (j ? a.rd ^ 16 : a.rd));

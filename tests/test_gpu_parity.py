@@ -457,6 +457,24 @@ def test_forward_decode_32_token_chunks(ctx, types, shape):
     assert st["path"] == 0 and st["chunk"] == 32 and st["max_group"] == max(sizes)
 
 
+@pytest.mark.parametrize("types", FORMATS, ids=lambda t: "/".join(W.TYPE_NAMES[x] for x in t))
+def test_decode_chunks_and_staging_same_bits(ctx, types):
+    """The decode kernels' ways to fetch and tile the activations give the same bits: one
+    expert over 33 tokens at once (32-token chunks, one whole and one of a single
+    token), in calls of 16 and 17 (one staged tile; a second tile of one token) and
+    token by token (direct loads, no LDS)."""
+    spec = dataclasses.replace(W.MIXTRAL_8X7B_Q4_0, name="one-expert", hidden=2048, inter=13312, n_experts=1, k=1,
+                               gate_type=types[0], up_type=types[1], down_type=types[2], scale_sigma=0.01)
+    layer = moe.MoeLayer(ctx, spec, synth.make_layer(spec, seed=67))
+    h, lg = synth.activations(spec, 33, seed=67), np.zeros((33, 1), np.float32)
+    whole, st = layer.forward(h, lg, stats=True)
+    assert st["path"] == 0 and st["chunk"] == 32
+    for cut in ([0, 16, 33], list(range(34))):
+        parts = [layer.forward(h[a:b], lg[a:b]) for a, b in zip(cut, cut[1:])]
+        assert np.array_equal(bits(np.concatenate(parts)), bits(whole)), cut
+    layer.free()
+
+
 @pytest.mark.parametrize("types", [(W.Q4_0, W.Q4_0, W.Q4_0), (W.Q4_K, W.Q4_K, W.Q6_K), (W.Q8_0, W.Q8_0, W.Q5_K)],
                          ids=lambda t: "/".join(W.TYPE_NAMES[x] for x in t))
 def test_forward_grouped_split_k_down(ctx, types):
