@@ -1205,6 +1205,7 @@ MmPlan plan_mm(int gate_type, int down_type, int H, int I, int P, int max_u, int
     // against 377 us on the DeepSeek 1024-token one: four wavefronts fetching the
     // same activations from L2 cost more than staging them once in LDS.)
     const long mean = P / std::max(max_u, 1);
+    bool lone = false;  // one wide group on the decode kernels
     const long pf_wgs = (long)((P + 63) / 64) * (I / 128);
     if (mean >= ANEDVD_STAGED_MIN && grouped_supported(H, I) && pf_wgs >= 256) {
         p.kind = kMmStaged;
@@ -1232,10 +1233,21 @@ MmPlan plan_mm(int gate_type, int down_type, int H, int I, int P, int max_u, int
         p.kind = kMmDecode;
         const size_t gu_bytes = (size_t)max_u * I * H / block_elems(gate_type) * block_bytes(gate_type) * 2;
         p.mt = mean >= kWideMean && gu_bytes >= kWideBytes ? 2 : 1;
+        lone = max_u == 1 && gu_bytes >= kWideBytes;
         p.stage = mean >= kStageMean;
     }
     p.chunk = 16 * p.mt;
-    p.nchunk = P / p.chunk + max_u;
+    // The list's capacity, and the grid's chunk columns: every group can leave one chunk
+    // partly filled.  The chunks of a lone group (one expert, a separate shared expert)
+    // are known exactly, and where it is wide an empty column costs more than anything
+    // else a chunk's size decides: at 32 tokens, in one 32-token chunk, Q4_0 H 4096
+    // I 14336 91.4 us with a second, empty column and 67.7 without (16-token chunks
+    // 83.6), Q6_K H 2048 I 5632 52.7 and 46.6 (49.5).  (Small lone experts gain and lose:
+    // Q4_K H = I = 2048 16 tokens 31.2 / 32.8, 64 tokens 44.3 / 39.2.  For more groups
+    // (P - max_u) / chunk + max_u would hold, but it moves which sizes give a multiple of
+    // 8 columns, where all workgroups of a chunk share an XCD: 32 F16 experts, 72 tokens,
+    // 50 columns 195 us, 48 220.)
+    p.nchunk = lone ? (P + p.chunk - 1) / p.chunk : P / p.chunk + max_u;
     p.xper = p.kind == kMmStaged && p.contig ? (p.nchunk + 7) / 8 : 0;  // the grouped grid's work items per XCD
     if (p.kind != kMmDecode) {
         p.ks_gu = 1;

@@ -475,6 +475,30 @@ def test_decode_chunks_and_staging_same_bits(ctx, types):
     layer.free()
 
 
+WIDE_LONE = [dataclasses.replace(W.MIXTRAL_8X7B_Q4_0, name="lone-expert", hidden=2048, inter=5632, n_experts=1, k=1,
+                                 gate_type=W.Q6_K, up_type=W.Q6_K, down_type=W.Q8_0, scale_sigma=0.01),
+             dataclasses.replace(W.MIXTRAL_8X7B_Q4_0, name="wide-separate-shared", hidden=2048, inter=256, n_experts=8,
+                                 gate_type=W.Q4_K, up_type=W.Q4_K, down_type=W.Q4_K, scale_sigma=0.01,
+                                 shared_inter=5632, shared_type=W.Q8_0, shared_gated=True)]
+
+
+@pytest.mark.parametrize("spec", WIDE_LONE, ids=lambda s: s.name)
+def test_forward_wide_lone_group(ctx, spec):
+    """A lone expert and a separate shared expert of 16 MB and more of gate and up: their
+    one group's work list holds exactly its chunks, at the edges of one and two 16-token
+    tiles and of whole 32-token chunks (the last of a full list must not be lost)."""
+    L = synth.make_layer(spec, seed=71)
+    layer = moe.MoeLayer(ctx, spec, L)
+    h, ol = synth.activations(spec, 97, seed=71), O.OracleLayer(spec, L)
+    lg = np.zeros((97, 1), np.float32) if spec.n_experts == 1 else ol.route(h, 97)[0]
+    want = ol.forward(h, lg, fast=True)
+    for T in (1, 15, 16, 17, 31, 32, 33, 64, 96, 97):
+        got, st = layer.forward(h[:T], lg[:T], stats=True)
+        err = moe.rel_l2(got, want[:T])
+        assert err <= REL_L2_TOL and st["path"] == 0, (T, err)
+    layer.free()
+
+
 @pytest.mark.parametrize("types", [(W.Q4_0, W.Q4_0, W.Q4_0), (W.Q4_K, W.Q4_K, W.Q6_K), (W.Q8_0, W.Q8_0, W.Q5_K)],
                          ids=lambda t: "/".join(W.TYPE_NAMES[x] for x in t))
 def test_forward_grouped_split_k_down(ctx, types):
