@@ -63,14 +63,32 @@ constexpr int kWaves = 4;
 #define ANEDVD_SMALL_MEAN 64
 #endif
 // Mean group size from which the decode kernels take 32-token chunks (two 16-token
-// tiles, the second skipped where a group has no tokens for it): most groups then
-// hold more than 16 tokens or nearly so, and each pass over an expert's weights serves
-// them all.  One box, 16- against 32-token chunks (us): Qwen3 Q8_0 mean 8 136.7 / 137.9,
-// mean 10 145.6 / 142.0, mean 16 200 / 161, mean 21 248 / 177; Q4_K_M mean 8 109.7 /
-// 113.8, mean 12 131.7 / 129.9, mean 21 205 / 156; Mixtral Q4_0 mean 10 203.2 / 204.4,
-// mean 25 368 / 281.  (64-token chunks: Qwen3 Q8_0 mean 21 186, the accumulators and
-// activations then leave one or two wavefronts per SIMD.)
-constexpr int kWideMean = 10;
+// tiles, the second skipped where a group has no tokens for it) instead of 16: the
+// groups past 16 tokens then stream their weights once, and pay for it with 1.5 times
+// the registers.  The line lies where the two cross, and that depends on what a second
+// stream costs.  Calls of 16- / 32-token chunks in us (128 experts of width 768, 32 of
+// 2048; hidden 2048; uniform routing):
+//   8 bits and more a weight, from 10: F16 mean 10 268 / 241 and 198 / 178; Q8_0 mean 10
+//     136 / 131 and 106 / 101, mean 12 147 / 137 and 106 / 108, mean 16 186 / 145.
+//   below, from 12: Q4_K (down Q6_K) mean 10 110 / 108 and 83 / 86, mean 12 118 / 116 and
+//     89 / 86, mean 14 125 / 120 and 95 / 92, mean 16 145 / 127; Q5_0 mean 10 113 / 112 and
+//     88 / 92, mean 12 122 / 120 and 93 / 93; Q5_1 mean 12 142 / 135 and 100 / 98; Q6_K mean
+//     10 124 / 125 and 96 / 98, mean 14 142 / 136 and 104 / 104; Q2_K and Q3_K mean 10 to 14
+//     within 1 %, mean 15 96 / 87; Q4_0 mean 12 82 / 78.
+//   Q5_K (172 and 198 VGPRs at two tiles, two wavefronts per SIMD), from 15: mean 10 122 /
+//     126 here and 92 / 96, mean 14 136 / 142 and 104 / 104, mean 15 147 / 146 and 111 / 104.
+//   gate/up's K split over workgroups (few experts: the call is short of workgroups and
+//     wider chunks halve them), from 16: 8 experts of width 2048, Q8_0 mean 12 52 / 57,
+//     mean 15 58 / 58, mean 16 71 / 65; Q6_K mean 12 48 / 53, mean 15 55 / 56, mean 18 62 /
+//     59; Q4_K mean 12 45 / 48, mean 16 55 / 54; F16 mean 12 72 / 78, mean 16 108 / 85.
+// A call of at most 16 tokens has no group for a second tile.  (64-token chunks: Qwen3
+// Q8_0 mean 21 186 us against 177, one or two wavefronts per SIMD.)
+static long wide_mean(int gate_type, bool split)
+{
+    if (split) return 16;
+    if (gate_type == ANEDVD_Q5_K) return 15;
+    return tile_fmt(gate_type).qb >= 16 ? 10 : 12;
+}
 // ... and the gate and up weights they read at least: below, a second pass over an
 // expert hits the L2s and half the workgroups only cost parallelism (the tiny layer,
 // 9 MB, 64 tokens 26.2 us at 16-token chunks, 28.2 at 32; the generic f16 layer with
@@ -80,7 +98,7 @@ constexpr size_t kWideBytes = (size_t)16 << 20;
 // Mean group size from which the decode kernels stage their activations (ASource):
 // with fewer tokens per group a direct load touches few lines anyway.
 constexpr int kStageMean = 2;
-static_assert(kStageMean <= kWideMean, "32-token chunks are staged");
+static_assert(kStageMean <= 10, "32-token chunks are staged");
 constexpr int kCUs = 256;  // MI355X compute units
 #ifdef ANEDVD_MM_WPE
 #define MM_ATTR __attribute__((amdgpu_waves_per_eu(ANEDVD_MM_WPE)))
@@ -1232,7 +1250,10 @@ MmPlan plan_mm(int gate_type, int down_type, int H, int I, int P, int max_u, int
     } else {
         p.kind = kMmDecode;
         const size_t gu_bytes = (size_t)max_u * I * H / block_elems(gate_type) * block_bytes(gate_type) * 2;
-        p.mt = mean >= kWideMean && gu_bytes >= kWideBytes ? 2 : 1;
+        p.ks_gu = choose_ks(H / kStep / steps_per_unit(gate_type), steps_per_unit(gate_type),
+                            (long)max_u * (I / kRowBlock), 2, 2);
+        const bool wide = T > 16 && gu_bytes >= kWideBytes && mean >= wide_mean(gate_type, p.ks_gu > 1);
+        p.mt = wide ? 2 : 1;
         lone = max_u == 1 && gu_bytes >= kWideBytes;
         p.stage = mean >= kStageMean;
     }
@@ -1253,8 +1274,6 @@ MmPlan plan_mm(int gate_type, int down_type, int H, int I, int P, int max_u, int
         p.ks_gu = 1;
         return p;
     }
-    p.ks_gu = choose_ks(H / kStep / steps_per_unit(gate_type), steps_per_unit(gate_type), (long)max_u * (I / kRowBlock),
-                        2, 2);
     p.ks_dn = choose_ks(I / kStep / steps_per_unit(down_type), steps_per_unit(down_type),
                         (long)max_u * ((H / kRowBlock + kWaves - 1) / kWaves), 1, 2);
 #ifdef ANEDVD_KS_DN

@@ -499,6 +499,33 @@ def test_forward_wide_lone_group(ctx, spec):
     layer.free()
 
 
+@pytest.mark.parametrize("t,E,k,H,I,sizes", [
+    (W.Q8_0, 1, 1, 2048, 5632, {10: 16, 15: 16, 16: 16, 17: 32, 31: 32, 33: 32}),     # one wide expert, K split
+    (W.Q8_0, 16, 12, 512, 4096, {13: 16, 14: 16, 16: 16, 17: 32}),                    # mean 9, 10, 12, 12
+    (W.Q8_0, 8, 2, 2048, 2048, {40: 16, 63: 16, 64: 32}),                             # few experts, K split
+    (W.Q6_K, 8, 2, 2048, 2048, {48: 16, 63: 16, 64: 32}),
+    (W.F16, 32, 4, 256, 2048, {79: 16, 80: 32}),                                      # mean 9, 10: K whole
+    (W.Q8_0, 32, 4, 256, 2048, {79: 16, 80: 32}),
+    (W.Q4_K, 32, 4, 256, 2048, {95: 16, 96: 32}),                                     # mean 11, 12
+    (W.Q5_0, 32, 4, 256, 2048, {95: 16, 96: 32}),
+    (W.Q5_K, 32, 4, 256, 2048, {119: 16, 120: 32}),                                   # mean 14, 15
+    (W.Q4_0, 8, 2, 512, 1024, {64: 16, 120: 16}),                                     # 9 MB of gate and up
+], ids=lambda v: "sizes" if isinstance(v, dict) else str(v))
+def test_decode_chunk_width(ctx, t, E, k, H, I, sizes):
+    """Which decode calls take 32-token chunks: never one of at most 16 tokens (no group
+    can have a second tile), and from the mean group size where each weight format, with
+    gate/up's K whole or split over workgroups, is the faster with them."""
+    spec = dataclasses.replace(W.MIXTRAL_8X7B_Q4_0, name="chunk-width", hidden=H, inter=I, n_experts=E, k=k,
+                               gate_type=t, up_type=t, down_type=t, scale_sigma=0.01)
+    layer = moe.MoeLayer(ctx, spec, synth.make_layer(spec, seed=73))
+    for T, chunk in sizes.items():
+        h, lg = synth.activations(spec, T, seed=73), np.zeros((T, E), np.float32)
+        lg[np.arange(T)[:, None], (np.arange(T)[:, None] * k + np.arange(k)) % E] = 1.0  # even groups
+        _, st = layer.forward(h, lg, stats=True)
+        assert st["path"] == 0 and st["chunk"] == chunk, (T, st)
+    layer.free()
+
+
 @pytest.mark.parametrize("types", [(W.Q4_0, W.Q4_0, W.Q4_0), (W.Q4_K, W.Q4_K, W.Q6_K), (W.Q8_0, W.Q8_0, W.Q5_K)],
                          ids=lambda t: "/".join(W.TYPE_NAMES[x] for x in t))
 def test_forward_grouped_split_k_down(ctx, types):
