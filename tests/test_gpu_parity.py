@@ -499,6 +499,23 @@ def test_forward_wide_lone_group(ctx, spec):
     layer.free()
 
 
+@pytest.mark.parametrize("types", FORMATS, ids=lambda t: "/".join(W.TYPE_NAMES[x] for x in t))
+def test_split_gateup_finish_same_bits(ctx, types):
+    """Gate/up's K partials finished inside the down kernel (calls of 16 tokens, 16-token
+    chunks) and by the reduction launch before the staged down (136 tokens over 8
+    experts, 32-token chunks: groups of 17) give the same bits."""
+    spec = dataclasses.replace(W.MIXTRAL_8X7B_Q4_0, name="split-finish", hidden=2048, inter=2048, n_experts=8, k=1,
+                               gate_type=types[0], up_type=types[1], down_type=types[2], scale_sigma=0.01)
+    layer = moe.MoeLayer(ctx, spec, synth.make_layer(spec, seed=79))
+    h, lg = synth.activations(spec, 136, seed=79), np.zeros((136, 8), np.float32)
+    lg[np.arange(136), np.arange(136) % 8] = 3.0
+    whole, st = layer.forward(h, lg, stats=True)
+    assert st["path"] == 0 and st["chunk"] == 32 and st["max_group"] == 17
+    parts = [layer.forward(h[a:a + 16], lg[a:a + 16]) for a in range(0, 136, 16)]
+    assert np.array_equal(bits(np.concatenate(parts)), bits(whole))
+    layer.free()
+
+
 @pytest.mark.parametrize("t,E,k,H,I,sizes", [
     (W.Q8_0, 1, 1, 2048, 5632, {10: 16, 15: 16, 16: 16, 17: 32, 31: 32, 33: 32}),     # one wide expert, K split
     (W.Q8_0, 16, 12, 512, 4096, {13: 16, 14: 16, 16: 16, 17: 32}),                    # mean 9, 10, 12, 12
