@@ -136,8 +136,9 @@ int ensure(Workspace &w, size_t bytes, hipStream_t st)
     return ANEDVD_OK;
 }
 
-// The host-pointer forward's pinned staging, grown on demand up to kPinMax and freed
-// with the context.  Caller memory is pageable: the runtime copies it through staging
+// The host-pointer forward's pinned staging, grown on demand (to a power of two, so that
+// prompts of growing length pin memory a few times and not once a call) up to kPinMax and
+// freed with the context.  Caller memory is pageable: the runtime copies it through staging
 // of its own or pins it page by page first (1 MB: 52 us in, 63 us out, 207 us out into
 // a fresh allocation), where pinned memory moves in 27 us and the host's own copies
 // take 12 us in and 35 us out (fresh).  False: larger than kPinMax, or no memory.
@@ -149,7 +150,8 @@ bool pinned_ensure(Workspace &w, size_t bytes)
     if (w.base) (void)hipHostFree(w.base);  // its last call ended with a synchronisation
     w.base = nullptr;
     w.cap = 0;
-    const size_t want = std::max(bytes, (size_t)1 << 20);
+    size_t want = (size_t)1 << 20;
+    while (want < bytes) want *= 2;  // at most kPinMax, itself a power of two
     if (hipHostMalloc(&w.base, want, hipHostMallocMapped) != hipSuccess) {
         (void)hipGetLastError();
         w.base = nullptr;

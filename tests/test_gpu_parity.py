@@ -656,6 +656,31 @@ def test_router_in_the_routing_launch_is_bit_exact(ctx, spec, Ts):
     layer.free()
 
 
+def test_host_forward_staging(ctx):
+    """forward() over host buffers against forward_device, bit for bit, on one context
+    whose staging grows, is larger than the call and is passed by: activations on both
+    sides of 256 KB (read by a kernel, copied), a logits block of no whole number of 16
+    bytes (7 experts), calls on both sides of the 64 MiB that the staging keeps, with
+    logits and with the layer's router."""
+    spec = dataclasses.replace(W.TINY_Q8_0, name="host-staging", n_experts=7)
+    layer = moe.MoeLayer(ctx, spec, synth.make_layer(spec, seed=83))
+    per = 2 * spec.hidden * 4 + spec.n_experts * 4  # staging bytes per token (h, out, logits)
+    most = ((64 << 20) - 32) // per
+    for T, given in [(3, True), (1, False), (127, True), (128, True), (129, True), (5, True), (1001, True), (64, False),
+                     (most, True), (most + 1, True), (most + 1, False), (9, True), (2048, False)]:
+        h = synth.activations(spec, T, seed=83 + T)
+        lg = synth.normal(5, T, T * 7).astype(np.float32).reshape(T, 7) if given else None
+        got = layer.forward(h, lg)
+        d_h, d_out = ctx.to_device(h), ctx.alloc(h.nbytes)
+        d_lg = ctx.to_device(lg) if given else None
+        layer.forward_device(d_h, T, d_lg, d_out)
+        ctx.synchronize()
+        assert np.array_equal(bits(got), bits(ctx.from_device(d_out, h.shape, np.float32))), (T, given)
+        for p in (d_h, d_out) + ((d_lg,) if given else ()):
+            ctx.free(p)
+    layer.free()
+
+
 def test_route_counts_match_the_routing(ctx):
     """Engine.route_counts through the drop-in (engine.zig:726-731, 1190-1195): after
     a forward call the layer's per-expert choices of that call are added to the
