@@ -46,6 +46,7 @@ struct anedvd_moe_ctx {
     Workspace ws;
     Workspace io;  // staging for the host-pointer entry points
     Workspace pin; // pinned host staging of the host-pointer forward (pinned_ensure)
+    void *pin_dev = nullptr;  // its address in kernels
     // The last forward call on this context (route counts read its dispatch).
     const anedvd_moe_layer *last_layer = nullptr;
     const int32_t *last_offsets = nullptr;
@@ -141,10 +142,12 @@ int ensure(Workspace &w, size_t bytes, hipStream_t st)
 // freed with the context.  Caller memory is pageable: the runtime copies it through staging
 // of its own or pins it page by page first (1 MB: 52 us in, 63 us out, 207 us out into
 // a fresh allocation), where pinned memory moves in 27 us and the host's own copies
-// take 12 us in and 35 us out (fresh).  False: larger than kPinMax, or no memory.
+// take 12 us in and 35 us out (fresh).  False: larger than kPinMax, or no memory
+// that kernels can reach; no error is left behind.
 constexpr size_t kPinMax = (size_t)64 << 20;
-bool pinned_ensure(Workspace &w, size_t bytes)
+bool pinned_ensure(anedvd_moe_ctx *c, size_t bytes)
 {
+    Workspace &w = c->pin;
     if (w.cap >= bytes) return true;
     if (bytes > kPinMax) return false;
     if (w.base) (void)hipHostFree(w.base);  // its last call ended with a synchronisation
@@ -153,8 +156,13 @@ bool pinned_ensure(Workspace &w, size_t bytes)
     size_t want = (size_t)1 << 20;
     while (want < bytes) want *= 2;  // at most kPinMax, itself a power of two
     if (hipHostMalloc(&w.base, want, hipHostMallocMapped) != hipSuccess) {
-        (void)hipGetLastError();
         w.base = nullptr;
+    } else if (hipHostGetDevicePointer(&c->pin_dev, w.base, 0) != hipSuccess) {
+        (void)hipHostFree(w.base);
+        w.base = nullptr;
+    }
+    if (!w.base) {
+        (void)hipGetLastError();  // the pageable path's launches must not report it
         return false;
     }
     w.cap = want;
@@ -1025,11 +1033,8 @@ int anedvd_moe_layer_forward(anedvd_moe_layer *L, const float *h, size_t T, cons
     const size_t hb = T * L->H * 4, lb = logits ? T * L->E * 4 : 0;
     const size_t l_at = (hb + 255) & ~(size_t)255, o_at = l_at + ((lb + 255) & ~(size_t)255),
                  m_at = o_at + ((hb + 255) & ~(size_t)255);
-    void *pd = nullptr;
-    const bool pin = pinned_ensure(L->ctx->pin, m_at + sizeof meta) &&
-                     hipHostGetDevicePointer(&pd, L->ctx->pin.base, 0) == hipSuccess;
-    if (pin) {
-        uint8_t *p = (uint8_t *)L->ctx->pin.base, *d = (uint8_t *)pd;
+    if (pinned_ensure(L->ctx, m_at + sizeof meta)) {
+        uint8_t *p = (uint8_t *)L->ctx->pin.base, *d = (uint8_t *)L->ctx->pin_dev;
         auto in = [&](const void *src, size_t at, size_t bytes, float *dst) -> int {
             memcpy(p + at, src, bytes);
             if (bytes > kPinKernelMax || bytes % 16) {
