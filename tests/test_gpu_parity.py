@@ -88,16 +88,21 @@ def test_resident_experts_bit_exact(ctx, types):
 @pytest.mark.parametrize("out_dim,in_dim,n", [(128, 2048, 1), (128, 2048, 64), (8, 512, 16), (64, 2048, 3),
                                               (7, 300, 5), (8, 4096, 2), (64, 2048, 1024), (128, 2048, 512),
                                               (100, 1003, 700), (8, 4096, 300), (70, 5, 3), (64, 2048, 1025),
-                                              (100, 1003, 5), (8, 64, 70000), (256, 1024, 300)])
+                                              (100, 1003, 5), (8, 64, 70000), (256, 1024, 300), (40, 1003, 65),
+                                              (100, 1003, 30), (7, 300, 70), (70, 5, 65), (1, 2048, 65),
+                                              (33, 4096, 65)])
 def test_matmul_f16_bit_exact(ctx, out_dim, in_dim, n):
-    """The router GEMV (cpu.matmulF16's chains) at the shapes of both launch forms:
-    a token and an expert per lane, and two of each (>= 64 experts and >= 32768
-    token-expert pairs: (64, 2048, 1024), (128, 2048, 512), and (100, 1003, 700) with
-    a partial second expert half and a partial last 8-j block plus a scalar tail; an
-    odd token count, whose last workgroup has one token), a hidden size below one
-    block (70, 5, 3), more token blocks than a grid's y dimension takes (8, 64,
-    70000: tokens run on x), and four 64-expert groups at two experts per lane (256,
-    1024, 300)."""
+    """The router GEMV (cpu.matmulF16's chains) at the shapes of its launch forms.  Two
+    tokens and two experts per lane (>= 64 experts and >= 32768 token-expert pairs):
+    (64, 2048, 1024), (128, 2048, 512), and (100, 1003, 700) with a partial second expert
+    half and a partial last 8-j block plus a scalar tail; an odd token count, whose last
+    workgroup has one token; four 64-expert groups (256, 1024, 300).  A token and an
+    expert per lane (more than 64 tokens or 2048 pairs below that): (40, 1003, 65) and
+    (100, 1003, 30) with a partial last 8-j block, a scalar tail and a partly filled last
+    block of 32 experts, (33, 4096, 65) with one expert in it, (7, 300, 70) and (1, 2048,
+    65) with wavefronts past the last expert, a hidden size below one block (70, 5, 65),
+    more token blocks than a grid's y dimension takes (8, 64, 70000: tokens run on x).
+    The other small calls run a wavefront per 8 experts and token (tested below)."""
     w = (synth.normal(1, out_dim, out_dim * in_dim) * 0.02).astype(np.float16).reshape(out_dim, in_dim)
     x = synth.normal(2, in_dim, n * in_dim).astype(np.float32).reshape(n, in_dim)
     got = ctx.matmul_f16(w, x)
@@ -447,7 +452,8 @@ def test_forward_grouped_every_live_tile_count(ctx, types):
 def test_forward_decode_32_token_chunks(ctx, types, shape):
     """The decode kernels' 32-token chunks (mean group 18, gate and up of 16 MB and
     more): groups at the edges of one and two 16-token tiles and of a second chunk, with
-    gate/up's K split (finished in the down kernel) and whole."""
+    gate/up's K split (finished by the reduction launch) and whole; the down kernel
+    stages its activations either way."""
     sizes = [1, 15, 16, 17, 31, 32, 33, 3]
     lg = _logits_for_groups(sizes, seed=31)
     spec = dataclasses.replace(W.MIXTRAL_8X7B_Q4_0, name="mm-32", hidden=shape[0], inter=shape[1],
@@ -625,27 +631,40 @@ def test_forward_grouped_small_groups(ctx, types):
     assert st["small_groups"] == sum(1 for n in SMALL_SIZES if n <= 16)
 
 
+def _router_in_routing(spec, T):
+    """The routing launch forms the logits itself: a chain per thread, a router (as f32)
+    that one CU streams, x in the dispatch's LDS (57.5 KB)."""
+    return (T <= 16 and T * spec.n_experts * 8 <= 1024 and spec.n_experts * spec.hidden * 4 <= 512 * 1024
+            and T * spec.hidden * 4 <= 56 * 1024)
+
+
+# (layer, calls that form their logits there, calls that are past a limit)
 ROUTER_IN_ROUTING = [
-    (dataclasses.replace(W.MIXTRAL_8X7B_Q4_0, name="mixtral-router", inter=256), (1, 2, 16)),
-    (dataclasses.replace(W.DEEPSEEK_V2_LITE_Q8_0, name="deepseek-router", inter=256, shared_inter=512), (1, 2)),
-    (dataclasses.replace(W.QWEN3_30B_A3B_Q8_0, name="qwen3-router", inter=256), (1,)),
-    (W.TINY_Q8_0, (1, 5, 16)),
+    (dataclasses.replace(W.MIXTRAL_8X7B_Q4_0, name="mixtral-router", inter=256), (1, 2), (16,)),
+    (dataclasses.replace(W.DEEPSEEK_V2_LITE_Q8_0, name="deepseek-router", inter=256, shared_inter=512), (1, 2), (3,)),
+    (dataclasses.replace(W.QWEN3_30B_A3B_Q8_0, name="128-experts-router", hidden=1024, inter=256), (1,), (2,)),
+    (dataclasses.replace(W.QWEN3_30B_A3B_Q8_0, name="qwen3-router", inter=256), (), (1,)),
+    (W.TINY_Q8_0, (1, 5, 16), (17,)),
 ]
 
 
-@pytest.mark.parametrize("spec,Ts", ROUTER_IN_ROUTING, ids=lambda v: v.name if hasattr(v, "name") else str(v))
-def test_router_in_the_routing_launch_is_bit_exact(ctx, spec, Ts):
+@pytest.mark.parametrize("spec,inside,outside", ROUTER_IN_ROUTING,
+                         ids=lambda v: v.name if hasattr(v, "name") else "-".join(map(str, v)) or "none")
+def test_router_in_the_routing_launch_is_bit_exact(ctx, spec, inside, outside):
     """A call of a few tokens without logits forms the router logits inside the
-    routing launch (a chain per thread, T E 8 <= 1024) instead of the router
-    GEMV launch: its output must equal, bit for bit, the same call given the
-    oracle's logits (cpu.matmulF16's order, which the router GEMV matches bit for
-    bit), so every logit bit is the same.  Shapes of Mixtral (H 4096, 8 experts),
-    DeepSeek-V2-Lite (64 experts and merged shared pieces), Qwen3 (128 experts at
-    one token) and the tiny layer (H 512: the largest T)."""
+    routing launch (a chain per thread, T E 8 <= 1024; a router of at most 512 KB as f32;
+    x in the dispatch's LDS) instead of a router launch: its output must equal, bit for
+    bit, the same call given the oracle's logits (cpu.matmulF16's order, which every
+    router kernel matches bit for bit), so every logit bit is the same.  Shapes of
+    Mixtral (H 4096, 8 experts), DeepSeek-V2-Lite (64 experts and merged shared pieces),
+    128 experts of H 1024 at one token (every thread a chain, two 64-expert groups, a
+    router of exactly 512 KB) and the tiny layer (H 512: the largest T), and of each a call
+    just past a limit; Qwen3's 1 MB router is past the size limit at any T."""
+    assert all(_router_in_routing(spec, T) for T in inside) and not any(_router_in_routing(spec, T) for T in outside)
     L = synth.make_layer(spec, seed=61)
     layer = moe.MoeLayer(ctx, spec, L)
     ol = O.OracleLayer(spec, L)
-    for T in Ts:
+    for T in inside + outside:
         h = synth.activations(spec, T, seed=61 + T)
         lg = ol.route(h, T)[0]
         fused = layer.forward(h)
