@@ -924,12 +924,12 @@ __global__ __launch_bounds__(256) void k_act_reduce(MmArgs a)
 // kAPart: gate/up split its K over KSg workgroups and left the partials in `part`.
 // The workgroup finishes the activations it reads itself, k_act_reduce's sums in
 // the same order (so the same bits), for its chunk's tokens and its K range only,
-// into LDS (dynamic: 16 rows of its steps, and their descales); the K loop then
+// into LDS (dynamic: 16 MT rows of its steps, and their descales); the K loop then
 // reads them from there.  No launch between gate/up and down.
 template <class D, int MT, ASource kSrc>
 __global__ __launch_bounds__(256) MM_ATTR void k_mm_down(MmArgs a)
 {
-    static_assert(kSrc != kAPart || MT == 1, "partials are finished here for 16-token chunks only");
+    static_assert(kSrc != kAPart || MT == 1 || D::kSpu == 1, "no plan has 64 pieces or fewer here");
     int e, p0, nt;
     if (!chunk_of<MT>(a.d, (int)(blockIdx.x % a.nchunk), e, p0, nt)) return;
     const int wv = wave_id(), lane = threadIdx.x & 63;
@@ -1180,14 +1180,31 @@ __global__ __launch_bounds__(256) void k_combine_rows(const float *__restrict__ 
 
 static int steps_per_unit(int type) { return tile_fmt(type).spu; }
 
-// Dynamic LDS of a kAPart down workgroup: 16 rows of its steps in the activation
+// Dynamic LDS of a kAPart down workgroup: 16 mt rows of its steps in the activation
 // format, and a descale per (step, row).
 constexpr size_t kFuseLdsMax = 64 * 1024;
-static size_t down_part_lds(int down_type, int I, int ks_dn)
+static size_t down_part_lds(int down_type, int I, int ks_dn, int mt)
 {
     const int spu = steps_per_unit(down_type);
     const size_t sw = (size_t)(I / kStep / spu / ks_dn) * spu;
-    return 16 * sw * 2 * kStep + sw * 16 * 4;
+    return mt * (16 * sw * 2 * kStep + sw * 16 * 4);
+}
+
+// Most bytes of partials that the down kernels of a call with 32-token chunks read to
+// finish gate/up themselves: every workgroup of a chunk's H / 256 row groups reads its K
+// range's partials, in front of its K loop.  Past it that costs more than k_act_reduce's
+// launch; later where the finishing kernel keeps three wavefronts per SIMD (152 and 162
+// VGPRs; Q8_0 170 against 164 staged, Q4_1, Q5_1 and F16 174 to 186).  Finished in the
+// down kernel / by the launch, us: 18 MB (16 experts, H 1024, I 512, 68 tokens) F16 38.3 /
+// 40.8, Q8_0 32.0 / 35.0, (32 experts, H 512, I 1024, 136 tokens) Q5_1 44.0 / 46.2; 25 MB
+// F16 44.0 / 44.5 and 62.1 / 64.5, Q8_0 36.4 / 38.8; 33 MB F16 51.6 / 49.7, Q8_0 43.0 /
+// 40.3; 36 MB Q8_0 44.6 / 42.6, Q4_0 40.1 / 43.1, Q5_0 42.3 / 44.5; 50 MB Q8_0 50.1 / 44.7,
+// Q5_1 54.3 / 50.0, Q4_0 45.6 / 46.7; 60 MB Q4_0 43.9 / 45.3, Q5_0 45.7 / 47.5; 65 MB Q4_0
+// 52.8 / 51.3, Q5_0 55.9 / 53.6; 77 MB (8 experts of 2048 x 2048, 74 tokens) Q8_0 67.1 /
+// 61.7, Q5_1 69.7 / 63.5, F16 86.2 / 84.6, Q4_0 58.5 / 55.7.
+static size_t fuse_reread(int down_type)
+{
+    return (size_t)(down_type == ANEDVD_Q4_0 || down_type == ANEDVD_Q5_0 ? 60 : 28) << 20;
 }
 
 bool mm_supported(int type) { return tile_fmt(type).qb != 0; }
@@ -1284,13 +1301,13 @@ MmPlan plan_mm(int gate_type, int down_type, int H, int I, int P, int max_u, int
     // a down workgroup's rows of its K range fit the LDS budget and its prologue
     // has at most 64 (token, step) pieces, four memory round trips (16 pieces each),
     // even if every token of the call sends a slot to the same expert (a chunk
-    // holds at most min(T, 16) tokens).  Otherwise, and for 32-token chunks,
-    // k_act_reduce finishes them: twice the pieces in front of every down workgroup's
-    // K loop cost more than the launch (8 experts of 2048 x 2048, 74 tokens, finished in
-    // the down kernel / by k_act_reduce: Q8_0 67.1 / 61.7 us, Q5_1 69.7 / 63.5, Q4_0 58.5 /
-    // 55.7, F16 86.2 / 84.6; Q4_K with twice the pieces allowed 63.5 / 54.9).
+    // holds at most min(T, 16 mt) tokens).  Otherwise k_act_reduce finishes them.  With
+    // 32-token chunks only types of one-step scale units have so few pieces (twice as many
+    // allowed, Q4_K at 8 experts of 2048 x 2048, 74 tokens: 63.5 against 54.9 us).
     const int sw = I / kStep / steps_per_unit(down_type) / p.ks_dn * steps_per_unit(down_type);
-    p.fuse = p.ks_gu > 1 && p.mt == 1 && down_part_lds(down_type, I, p.ks_dn) <= kFuseLdsMax && std::min(T, 16) * sw <= 64;
+    const size_t reread = (size_t)P * I * 8 * p.ks_gu * ((H / kRowBlock + kWaves - 1) / kWaves);
+    p.fuse = p.ks_gu > 1 && (p.mt == 1 || reread <= fuse_reread(down_type)) &&
+             down_part_lds(down_type, I, p.ks_dn, p.mt) <= kFuseLdsMax && std::min(T, p.chunk) * sw <= 64;
     return p;
 }
 
@@ -1309,7 +1326,7 @@ template <class D, int MT, ASource kSrc>
 static int launch_down_t(const MmArgs &a, hipStream_t st)
 {
     const size_t wgs = (size_t)a.nchunk * ((a.H / kRowBlock + kWaves - 1) / kWaves) * a.KS;
-    const size_t lds = kSrc == kAPart ? down_part_lds(a.w0.type, a.I, a.KS) : 0;
+    const size_t lds = kSrc == kAPart ? down_part_lds(a.w0.type, a.I, a.KS, MT) : 0;
     hipLaunchKernelGGL((k_mm_down<D, MT, kSrc>), dim3((unsigned)wgs), dim3(256), lds, st, a);
     ANEDVD_HIP(hipGetLastError());
     return ANEDVD_OK;
@@ -1325,7 +1342,10 @@ static int launch_gateup_d(const MmArgs &a, const MmPlan &p, hipStream_t st)
 template <class D>
 static int launch_down_d(const MmArgs &a, const MmPlan &p, hipStream_t st)
 {
-    if (p.mt == 2) return launch_down_t<D, 2, kAStaged>(a, st);  // plan_mm: no fused finish
+    if constexpr (D::kSpu == 1) {  // plan_mm fuses no others at two tiles
+        if (a.KSg > 1 && p.mt == 2) return launch_down_t<D, 2, kAPart>(a, st);
+    }
+    if (p.mt == 2) return launch_down_t<D, 2, kAStaged>(a, st);
     if (a.KSg > 1) return launch_down_t<D, 1, kAPart>(a, st);
     return p.stage ? launch_down_t<D, 1, kAStaged>(a, st) : launch_down_t<D, 1, kASelf>(a, st);
 }

@@ -505,12 +505,17 @@ def test_forward_wide_lone_group(ctx, spec):
     layer.free()
 
 
-@pytest.mark.parametrize("types", FORMATS, ids=lambda t: "/".join(W.TYPE_NAMES[x] for x in t))
-def test_split_gateup_finish_same_bits(ctx, types):
-    """Gate/up's K partials finished inside the down kernel (calls of 16 tokens, 16-token
-    chunks) and by the reduction launch before the staged down (136 tokens over 8
-    experts, 32-token chunks: groups of 17) give the same bits."""
-    spec = dataclasses.replace(W.MIXTRAL_8X7B_Q4_0, name="split-finish", hidden=2048, inter=2048, n_experts=8, k=1,
+@pytest.mark.parametrize("types,H,I", [(t, 2048, 2048) for t in FORMATS] + [(t, 768, 2048) for t in
+                                                                          ((W.Q8_0,) * 3, (W.F16,) * 3, (W.Q5_1,) * 3,
+                                                                           (W.Q5_0,) * 3)],
+                         ids=lambda v: "/".join(W.TYPE_NAMES[x] for x in v) if isinstance(v, tuple) else str(v))
+def test_split_gateup_finish_same_bits(ctx, types, H, I):
+    """Gate/up's K partials finished inside the down kernel at 16-token chunks (calls of
+    16 tokens) and, with 136 tokens over 8 experts (32-token chunks, groups of 17), by the
+    reduction launch before the staged down (H = I = 2048: 71 MB of partials read again) or
+    inside the down kernel (H 768, types of one-step scale units: 20 MB) give the
+    same bits."""
+    spec = dataclasses.replace(W.MIXTRAL_8X7B_Q4_0, name="split-finish", hidden=H, inter=I, n_experts=8, k=1,
                                gate_type=types[0], up_type=types[1], down_type=types[2], scale_sigma=0.01)
     layer = moe.MoeLayer(ctx, spec, synth.make_layer(spec, seed=79))
     h, lg = synth.activations(spec, 136, seed=79), np.zeros((136, 8), np.float32)
