@@ -65,8 +65,10 @@ constexpr int kWaves = 4;
 // Mean group size from which the decode kernels take 32-token chunks (two 16-token
 // tiles, the second skipped where a group has no tokens for it) instead of 16: the
 // groups past 16 tokens then stream their weights once, and pay for it with 1.5 times
-// the registers.  The line lies where the two cross, and that depends on what a second
-// stream costs.  Calls of 16- / 32-token chunks in us (128 experts of width 768, 32 of
+// the registers (VGPRs of the staged gate/up and down kernels, 16 / 32 tokens: Q8_0 99 /
+// 147 and 110 / 163, four / three wavefronts per SIMD; at two wavefronts Q5_K and F16 in
+// both, Q6_K 169 in gate/up and the super-block types and Q5_1 in down).  The line lies
+// where the two cross, and that depends on what a second stream costs.  Calls of 16- / 32-token chunks in us (128 experts of width 768, 32 of
 // 2048; hidden 2048; uniform routing):
 //   8 bits and more a weight, from 10: F16 mean 10 268 / 241 and 198 / 178; Q8_0 mean 10
 //     136 / 131 and 106 / 101, mean 12 147 / 137 and 106 / 108, mean 16 186 / 145.
@@ -89,6 +91,7 @@ static long wide_mean(int gate_type, bool split)
     if (gate_type == ANEDVD_Q5_K) return 15;
     return tile_fmt(gate_type).qb >= 16 ? 10 : 12;
 }
+
 // ... and the gate and up weights they read at least: below, a second pass over an
 // expert hits the L2s and half the workgroups only cost parallelism (the tiny layer,
 // 9 MB, 64 tokens 26.2 us at 16-token chunks, 28.2 at 32; the generic f16 layer with
@@ -1233,7 +1236,8 @@ MmPlan plan_mm(int gate_type, int down_type, int H, int I, int P, int max_u, int
     // shared by four wavefronts) once the groups average 32 tokens and its gate/up
     // grid has a workgroup per CU at least; the chunks then give the grid its
     // parallelism and K is not split.  Below that, the decode kernels: chunks of one
-    // or two 16-token tiles, activations straight from L2, K split over workgroups.  (A single
+    // or two 16-token tiles, activations from L2 by each wavefront for itself (through its
+    // own LDS from a mean of two tokens on), K split over workgroups.  (A single
     // shared expert at 32 tokens on the grouped GEMM would be 22 workgroups: it
     // measured 105 us against the decode kernels' split K.  Kernels that read the
     // activations from L2 per wavefront with folded scales and 32- or 64-token

@@ -235,9 +235,9 @@ __global__ __launch_bounds__(256) void k_router(const float *__restrict__ wt, co
 // flight.  The call is bound by the latency of its weight loads and by what one CU
 // streams: k_router's 32-expert blocks read 256 KB each (Qwen3) two blocks ahead, the
 // fused routing workgroup the whole megabyte.  Here 16 CUs read 64 KB each.  Routing
-// stage with a cold router, k_router or fused / this kernel (us): Qwen3 1 token 21.4 /
-// 14.9, 7 tokens 17.4 / 15.0, 16 tokens 17.3 / 16.2; DeepSeek-V2-Lite 4 tokens 15.2 /
-// 13.5, 32 tokens 17.0 / 16.0.
+// stage with a cold router (us): Qwen3 1 token 21.4 in the routing workgroup / 14.9 here;
+// k_router / here: 7 tokens 17.4 / 15.0, 16 tokens 17.3 / 16.2, DeepSeek-V2-Lite 4 tokens
+// 15.2 / 13.5, 32 tokens 17.0 / 16.0.
 __global__ __launch_bounds__(64) void k_router_wave(const float *__restrict__ wt, const uint16_t *__restrict__ w,
                                                     const float *__restrict__ x, int E, int H,
                                                     float *__restrict__ logits)
@@ -322,12 +322,18 @@ int launch_router(const float *d_wt, const uint16_t *d_w, const float *d_x, int 
     // Two tokens and two experts per lane once the grid still has about one
     // wavefront per SIMD that way (Qwen3 333 tokens 11.4 against 14.9 us at one and one,
     // 256 tokens 10.6 / 10.8, 192 tokens 10.7 / 8.9, DeepSeek-V2-Lite 768 tokens 11.8 /
-    // 15.4; Qwen3 512 tokens and DeepSeek-V2-Lite 1024 11.5 and 11.8 us against 13.1 and
+    // 15.4; layer calls, two and two / one and one: 64 experts 512 tokens 108.7 / 108.8, 256
+    // experts 128 tokens 83.6 / 84.0, of H 7168 260 / 256 and at 140 tokens 260 / 263, 160
+    // experts of H 5120 at 225 tokens 179 / 178, at 256 tokens 184 / 185; Qwen3 512 tokens and DeepSeek-V2-Lite 1024 11.5 and 11.8 us against 13.1 and
     // 13.4 at one expert); one of each below (64 tokens of 128 experts: 5.1 against
     // 6.3 us at two tokens), and one expert for E < 64 (Mixtral's E = 8).
     const bool big = E >= 64 && (long)T * E >= 32768;
-    // A few tokens: one wavefront per 8 experts and token (up to 2048 (token, expert)
-    // pairs; 32 tokens of 128 experts: 17.1 against 17.9 us).
+    // A few tokens: one wavefront per 8 experts and token.  Up to 2048 (token, expert)
+    // pairs it is the faster, at twice that the slower: layer calls with k_router<1, 1> /
+    // k_router_wave, 128 experts 16 tokens 43.4 / 43.1 us, 24 tokens 45.2 / 45.4, 32 tokens
+    // 47.1 / 47.7; 64 experts 32 tokens 41.4 / 40.3, 48 tokens 43.5 / 43.5; 256 experts 4
+    // tokens 32.3 / 31.6, 8 tokens 35.7 / 35.8; 8 experts of H 4096, 64 tokens 48.9 / 47.7,
+    // 96 tokens 50.8 / 51.8.
     const size_t wave_lds = (size_t)8 * router_stride(H >> 3) * 4;
     if (T <= 64 && (long)T * E <= 2048 && wave_lds <= 65536) {
         hipLaunchKernelGGL(k_router_wave, dim3((unsigned)((E + 7) / 8), (unsigned)T), dim3(64), wave_lds, st, d_wt, d_w,

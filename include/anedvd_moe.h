@@ -86,10 +86,10 @@ typedef struct {
     uint32_t touched_experts;      /* experts with >= 1 routed token in this call */
     uint64_t weight_bytes;         /* expert + shared + router bytes the call had to read */
     uint32_t max_group;            /* largest tokens-per-expert group */
-    uint32_t path;                 /* expert kernels: 0 = decode (16-token tiles), 1 = grouped GEMM */
+    uint32_t path;                 /* expert kernels: 0 = decode (one or two 16-token tiles), 1 = grouped GEMM */
     uint32_t chunk;                /* tokens per expert-kernel work item: 16, 32, 64 or 128 */
     uint32_t down_ks;              /* K shares of the down product (partial planes the combine adds) */
-    uint32_t small_groups;         /* grouped GEMM calls: groups of <= 16 tokens run on the decode kernels */
+    uint32_t small_groups;         /* grouped GEMM calls: groups of <= 16 tokens, on one 16-token tile each */
 } anedvd_moe_stats;
 
 /* ------------------------------------------------------------------ lifetime */

@@ -638,9 +638,9 @@ def test_forward_grouped_small_groups(ctx, types):
 
 def _router_in_routing(spec, T):
     """The routing launch forms the logits itself: a chain per thread, a router (as f32)
-    that one CU streams, x in the dispatch's LDS (57.5 KB)."""
+    that one CU streams, x in the dispatch's LDS (35 KB)."""
     return (T <= 16 and T * spec.n_experts * 8 <= 1024 and spec.n_experts * spec.hidden * 4 <= 512 * 1024
-            and T * spec.hidden * 4 <= 56 * 1024)
+            and T * spec.hidden * 4 <= 35 * 1024)
 
 
 # (layer, calls that form their logits there, calls that are past a limit)
